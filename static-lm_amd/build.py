@@ -23,7 +23,7 @@ HOST_DEMO = PKG_DIR / "slm_host_demo"
 BUILD_DIR = PKG_DIR / "_build"
 
 HIP_SOURCES = ["slm_attn.hip", "slm_layer.hip", "slm_model.hip", "rope_append.hip",
-               "attn_decode.hip", "prefill_mfma.hip", "quant_gemm.hip", "norm_act.hip"]
+               "attn_decode.hip", "prefill_mfma.hip", "prefill_split.hip", "quant_gemm.hip", "norm_act.hip"]
 # measurement probes of the bench, a library of their own (not the product's)
 CALIB_DIR = PKG_DIR / "calib"
 CALIB_LIB = CALIB_DIR / "libslm_calib.so"
@@ -49,7 +49,8 @@ HIP_FLAGS = [
 # per-source extras: the Q4_0 GEMM's MFMA results go straight to VGPRs (its
 # epilogue reads every one; accumulator registers would cost a
 # v_accvgpr_read per element)
-HIP_SOURCE_FLAGS = {"quant_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+HIP_SOURCE_FLAGS = {"quant_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+                    "prefill_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
 def _run(cmd: list[str]) -> None:

@@ -6,11 +6,9 @@
 // Tiling.  A workgroup of HW*QS waves owns one query block and HW query heads
 // of one KV head (HW divides kv_mul), so every K/V tile staged in LDS serves
 // HW*QS waves.  Each wave owns 16*NQT query rows of one head.  Keys stream
-// through LDS in tiles of 32 rows.  For hd 128 with four heads per KV head
-// (the Llama-3-8B shape) eight waves share each tile and the tiles go from
-// memory straight into two LDS buffers (buffer loads with the lds bit), with
-// no registers held for the next tile, four waves per SIMD; otherwise the
-// next tile is prefetched into registers while the current one is in use.
+// through LDS in tiles of 32 rows, the next tile prefetched into registers
+// while the current one is in use.  (Most hd-128 batches run on bf16 matrix
+// cores instead, prefill_split.hip.)
 //
 // Transposed products keep softmax state lane-local.  With the 16x16x4 MFMA
 // layout (lane l: A[l%16][l/16], B[l/16][l%16], D[4*(l/16)+r][l%16]):
@@ -29,11 +27,9 @@
 // running sum stays a per-lane partial until the end.
 //
 // Which form of the kernel a batch runs (heads and blocks per workgroup,
-// paired blocks, key splits, DMA-fed tiles) is decided in prefill_plan.h,
-// with the measurements behind each rule.
+// paired blocks, key splits) is decided in prefill_plan.h, with the
+// measurements behind each rule.
 #include <math.h>
-
-#include <type_traits>
 
 #include "attn_common.h"
 #include "prefill_plan.h"
@@ -108,21 +104,6 @@ struct PrefillLds<256> {
     static __device__ __forceinline__ int k_swz(int) { return 0; }
 };
 
-// Tiles written by buffer->LDS DMA (hd 128): a wave's DMA instruction fills
-// 1 KiB of LDS contiguously, so rows cannot be padded.  Rows are 128 floats;
-// the K chunk index is XORed with k_swz(row) (bits 0-1 and 3 of the row), and
-// lane m reads its two V chunks in the order vrot(m).  Checked conflict-free
-// under the rule above on the CPU, for both readings of the lane grouping.
-template <int HD>
-struct PrefillLdsDma;
-template <>
-struct PrefillLdsDma<128> {
-    static constexpr int LDK = 128;
-    static constexpr int LDV = 128;
-    static __device__ __forceinline__ int k_swz(int r) { return (r & 3) | (((r >> 3) & 1) << 2); }
-    static __device__ __forceinline__ int vrot(int m) { return (m >> 3) & 1; }
-};
-
 // First 128-bit chunk lane m reads of its NDT contiguous V dims (NDT a
 // multiple of 4; lane m starts at float m*NDT of its row): with the V row
 // strides above, every cycle's 16 lanes then cover the 64 banks once.
@@ -140,11 +121,7 @@ constexpr int prefill_waves_per_simd() {
     return HD > 128 ? 1 : 2;
 }
 
-// DMA: K/V tiles go straight from memory to LDS (buffer loads with the lds
-// bit) into two buffers, with no registers held for the next tile; four waves
-// per SIMD.  Otherwise the next tile is prefetched into registers.
-//
-// KSP (register prefetch only): key splits.  The workgroup holds KSP sets of
+// KSP: key splits.  The workgroup holds KSP sets of
 // HW*QS waves; set k attends tiles k, k + KSP, k + 2*KSP, ... of its query
 // block, the KSP tiles of a step loaded together into KSP LDS slots, and at
 // the end sets 1..KSP-1 hand their (max, sum, O) to set 0 through LDS, which
@@ -159,16 +136,15 @@ constexpr int prefill_waves_per_simd() {
 // waves are numbered key split first, then head, then block: the waves of one
 // SIMD hold the same head and key split of the heavy and the light block,
 // and every SIMD gets the same share.
-template <int HD, int HW, int QS, int NQT, int kKT = 32, int NB = 1, bool PRIO = false,
-          bool DMA = false, int KSP = 1, bool PAIR = false>
-__global__ __launch_bounds__(64 * HW * QS * KSP,
-                             (DMA ? 4 : prefill_waves_per_simd<HD, HW>())) void
+template <int HD, int HW, int QS, int NQT, int KSP, bool PAIR>
+__global__ __launch_bounds__(64 * HW * QS * KSP, (prefill_waves_per_simd<HD, HW>())) void
 prefill_mfma_kernel(PrefillParams p) {
+    constexpr int kKT = 32;
     constexpr int KS = kKT / 16;  // 16-key sub-tiles per LDS tile
     constexpr int NWS = HW * QS;  // waves of one key split
     constexpr int NW = NWS * KSP;
     constexpr int NT = 64 * NW;
-    using Lds = std::conditional_t<DMA, PrefillLdsDma<HD>, PrefillLds<HD>>;
+    using Lds = PrefillLds<HD>;
     constexpr int LDK = Lds::LDK;
     constexpr int LDV = Lds::LDV;
     constexpr int DPL = HD / 4;   // contiguous head dims per lane group
@@ -186,13 +162,10 @@ prefill_mfma_kernel(PrefillParams p) {
     constexpr bool VEC_V = NDT % 4 == 0;
     constexpr int VC = VEC_V ? NDT / 4 : 1;
 
-    // NB LDS buffers: with two, a tile is stored while the other is read and
-    // one barrier per tile suffices.  With key splits, KSP tile slots (one
-    // buffer each), in one array so the merge at the end can reuse it whole.
-    static_assert(!DMA || NB == 2, "DMA tiles use two buffers");
-    static_assert(KSP == 1 || (!DMA && NB == 1), "key splits: register prefetch, one buffer");
+    // One LDS tile buffer per key split, in one array so the merge at the end
+    // can reuse it whole.
     static_assert(KSP == 1 || F4 % 64 == 0, "key splits: a wave's tile loads in one slot");
-    constexpr int NSLOT = NB * KSP;
+    constexpr int NSLOT = KSP;
     __shared__ __align__(16) float s_tiles[NSLOT * kKT * (LDK + LDV)];
     float(*sKb)[kKT * LDK] = reinterpret_cast<float(*)[kKT * LDK]>(s_tiles);
     float(*sVb)[kKT * LDV] = reinterpret_cast<float(*)[kKT * LDV]>(s_tiles + NSLOT * kKT * LDK);
@@ -297,15 +270,9 @@ prefill_mfma_kernel(PrefillParams p) {
         for (int dt = 0; dt < NDT; ++dt) o[qt][dt] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
 
-    auto vrot_of = [](int m) {
-        if constexpr (DMA)
-            return Lds::vrot(m);
-        else
-            return v_rot<NDT>(m);
-    };
     int v_off[VC];  // this lane's chunk offsets inside its NDT dims
 #pragma unroll
-    for (int c = 0; c < VC; ++c) v_off[c] = 4 * ((c + vrot_of(lr)) % VC);
+    for (int c = 0; c < VC; ++c) v_off[c] = 4 * ((c + v_rot<NDT>(lr)) % VC);
 
     const float* kg = p.k_cache + g * HD;
     const float* vg = p.v_cache + g * HD;
@@ -317,26 +284,11 @@ prefill_mfma_kernel(PrefillParams p) {
     // the loop costs MFMA time).  The descriptor's range ends at row kv_len,
     // and buffer loads past the range return zeros: the rows past the end
     // read as zeros without a branch.
-    constexpr int NI = DMA ? F4 / NT : 1;  // DMA instructions per wave, tile and matrix
-    static_assert(!DMA || F4 % NT == 0, "DMA tiles: whole instructions per wave");
-    int t_off[DMA ? 1 : NPF];
-    int d_off_k[NI], d_off_v[NI];
-    if constexpr (DMA) {
-        // instruction i of this wave fills float4 slots (wave*NI + i)*64 + lane
-        // of a tile; K slot (row r, chunk c) receives chunk c ^ k_swz(r)
+    int t_off[NPF];
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            const int f = (wave * NI + i) * 64 + lane;
-            const int r = f / (HD / 4), c = f % (HD / 4);
-            d_off_k[i] = (r * p.kv_dim + 4 * (c ^ Lds::k_swz(r))) * 4;
-            d_off_v[i] = (r * p.kv_dim + 4 * c) * 4;
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < NPF; ++i) {
-            const int f = (tid + i * NT) % F4;  // within its tile slot
-            t_off[i] = ((f / (HD / 4)) * p.kv_dim + (f % (HD / 4)) * 4) * 4;
-        }
+    for (int i = 0; i < NPF; ++i) {
+        const int f = (tid + i * NT) % F4;  // within its tile slot
+        t_off[i] = ((f / (HD / 4)) * p.kv_dim + (f % (HD / 4)) * 4) * 4;
     }
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
     auto bload = [](__amdgpu_buffer_rsrc_t r, int off) {
@@ -344,7 +296,7 @@ prefill_mfma_kernel(PrefillParams p) {
         return make_float4(__uint_as_float(x.x), __uint_as_float(x.y), __uint_as_float(x.z),
                            __uint_as_float(x.w));
     };
-    float4 pk[DMA ? 1 : NPF], pv[DMA ? 1 : NPF];
+    float4 pk[NPF], pv[NPF];
     static_assert(tile_range_fits(kKT, kMaxKvDim), "tile ranges must fit 32 bits");
     // Register prefetch of the KSP tiles from tile kt0: this thread's float4 i
     // belongs to slot (wave*64 + i*NT) / F4 (whole waves per slot, so the
@@ -385,44 +337,10 @@ prefill_mfma_kernel(PrefillParams p) {
             }
         }
     };
-    auto prefetch = [&](int kb, int buf) __attribute__((always_inline)) {
-        // rows kb .. min(kv_len, kb + kKT) - 1: bounded by the tile (one
-        // layer's K slice may pass 4 GiB)
-        const int bytes = (int)tile_range_bytes(kv_len, kb, kKT, p.kv_dim);
-        const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<float*>(kg + (long)kb * p.kv_dim), 0, bytes, 0x00020000);
-        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<float*>(vg + (long)kb * p.kv_dim), 0, bytes, 0x00020000);
-        if constexpr (DMA) {
-            // Issued as inline assembly: the compiler then sees no LDS store
-            // here, so it does not make the current tile's LDS reads wait for
-            // this DMA (it cannot tell the two buffers apart); the vmcnt(0)
-            // wait and the barrier ahead of the next tile order them instead.
-            // M0 holds the wave's LDS destination; lane l's 16 bytes land at
-            // M0 + 16*l.
-#pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                const unsigned lk = (unsigned)(unsigned long)(
-                    __attribute__((address_space(3))) float*)&sKb[buf][(wave * NI + i) * 256];
-                const unsigned lv = (unsigned)(unsigned long)(
-                    __attribute__((address_space(3))) float*)&sVb[buf][(wave * NI + i) * 256];
-                asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(d_off_k[i]),
-                             "s"(rk), "{m0}"(lk) : "memory");
-                asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(d_off_v[i]),
-                             "s"(rv), "{m0}"(lv) : "memory");
-            }
-        } else {
-            (void)buf;  // register prefetch goes through prefetch_regs
-            (void)rk;
-            (void)rv;
-        }
-    };
-
     // One key tile: S^T = K.Q^T, causal mask, online softmax, O^T += V^T.P^T.
     auto attend = [&](int kb, const float* sK, const float* sV) __attribute__((always_inline)) {
         // S^T tiles [key sub-tile][query tile]; the KS*NQT accumulators are
         // updated round-robin so consecutive MFMAs never depend on each other
-        if (PRIO) __builtin_amdgcn_s_setprio(1);
         floatx4 s[KS][NQT];
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
@@ -447,7 +365,6 @@ prefill_mfma_kernel(PrefillParams p) {
             }
         }
 
-        if (PRIO) __builtin_amdgcn_s_setprio(0);
 
         // causal mask, online softmax
         const bool diag = kb + kKT - 1 > p.start + q0;  // some key may be masked
@@ -511,7 +428,6 @@ prefill_mfma_kernel(PrefillParams p) {
         }
 
         // O^T += V^T . P^T
-        if (PRIO) __builtin_amdgcn_s_setprio(1);
         if constexpr (VEC_V) {
             // row m of every O^T tile belongs to lane m: its NDT head dims are
             // contiguous, read as 128-bit chunks in the lane's rotated order
@@ -551,71 +467,46 @@ prefill_mfma_kernel(PrefillParams p) {
                 }
             }
         }
-        if (PRIO) __builtin_amdgcn_s_setprio(0);
     };
 
-    if constexpr (DMA)
-        prefetch(0, 0);
-    else
-        prefetch_regs(0);
-    if constexpr (DMA) {
-        // Two tiles per trip, so each tile's buffer is a compile-time constant:
-        // the LDS read addresses are then loop-invariant registers plus
-        // immediate offsets instead of being recomputed per tile.
-        auto step = [&](int it, auto buf_c) __attribute__((always_inline)) {
-            constexpr int buf = decltype(buf_c)::value;
-            // this wave's DMA of tile it has landed; after the barrier every
-            // wave's has, and every wave is done with the other buffer
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __syncthreads();
-            if (it + 1 < n_tiles) prefetch((it + 1) * kKT, buf ^ 1);
-            const int kb = it * kKT;
-            if (wave_rows == 0 || kb > wave_last_pos) return;  // wave-uniform
-            attend(kb, sKb[buf], sVb[buf]);
-        };
-        for (int it = 0; it < n_tiles; it += 2) {
-            step(it, std::integral_constant<int, 0>());
-            if (it + 1 < n_tiles) step(it + 1, std::integral_constant<int, 1>());
-        }
-    } else {
-        // step st: tiles st*KSP .. st*KSP + KSP - 1 in slots 0..KSP-1; key
-        // split kspl attends slot kspl
-        const int n_steps = (n_tiles + KSP - 1) / KSP;
-        for (int st = 0; st < n_steps; ++st) {
-            const int kt0 = st * KSP;
-            if (NB == 1) __syncthreads();  // every wave is done with the previous tiles
+    prefetch_regs(0);
+    // step st: tiles st*KSP .. st*KSP + KSP - 1 in slots 0..KSP-1; key
+    // split kspl attends slot kspl
+    const int n_steps = (n_tiles + KSP - 1) / KSP;
+    for (int st = 0; st < n_steps; ++st) {
+        const int kt0 = st * KSP;
+        __syncthreads();  // every wave is done with the previous tiles
 #pragma unroll
-            for (int i = 0; i < NPF; ++i) {
-                const int f = tid + i * NT;
-                if constexpr (KSP == 1) {
-                    if (f < F4) {
-                        const int r = f / (HD / 4), ch = f % (HD / 4);
-                        float* sK = sKb[st % NB];
-                        float* sV = sVb[st % NB];
-                        *reinterpret_cast<float4*>(&sK[r * LDK + 4 * (ch ^ Lds::k_swz(r))]) =
-                            pk[i];
-                        *reinterpret_cast<float4*>(&sV[r * LDV + 4 * ch]) = pv[i];
-                    }
-                } else {
-                    const int slot = (wave * 64 + i * NT) / F4;  // uniform
-                    if (f < F4 * KSP && kt0 + slot < n_tiles) {
-                        const int fr = f % F4;
-                        const int r = fr / (HD / 4), ch = fr % (HD / 4);
-                        float* sK = sKb[(st % NB) * KSP + slot];
-                        float* sV = sVb[(st % NB) * KSP + slot];
-                        *reinterpret_cast<float4*>(&sK[r * LDK + 4 * (ch ^ Lds::k_swz(r))]) =
-                            pk[i];
-                        *reinterpret_cast<float4*>(&sV[r * LDV + 4 * ch]) = pv[i];
-                    }
+        for (int i = 0; i < NPF; ++i) {
+            const int f = tid + i * NT;
+            if constexpr (KSP == 1) {
+                if (f < F4) {
+                    const int r = f / (HD / 4), ch = f % (HD / 4);
+                    float* sK = sKb[0];
+                    float* sV = sVb[0];
+                    *reinterpret_cast<float4*>(&sK[r * LDK + 4 * (ch ^ Lds::k_swz(r))]) =
+                        pk[i];
+                    *reinterpret_cast<float4*>(&sV[r * LDV + 4 * ch]) = pv[i];
+                }
+            } else {
+                const int slot = (wave * 64 + i * NT) / F4;  // uniform
+                if (f < F4 * KSP && kt0 + slot < n_tiles) {
+                    const int fr = f % F4;
+                    const int r = fr / (HD / 4), ch = fr % (HD / 4);
+                    float* sK = sKb[slot];
+                    float* sV = sVb[slot];
+                    *reinterpret_cast<float4*>(&sK[r * LDK + 4 * (ch ^ Lds::k_swz(r))]) =
+                        pk[i];
+                    *reinterpret_cast<float4*>(&sV[r * LDV + 4 * ch]) = pv[i];
                 }
             }
-            __syncthreads();
-            if (st + 1 < n_steps) prefetch_regs(kt0 + KSP);
-            const int it = kt0 + kspl;
-            const int kb = it * kKT;
-            if (it >= n_tiles || wave_rows == 0 || kb > wave_last_pos) continue;  // uniform
-            attend(kb, sKb[(st % NB) * KSP + kspl], sVb[(st % NB) * KSP + kspl]);
         }
+        __syncthreads();
+        if (st + 1 < n_steps) prefetch_regs(kt0 + KSP);
+        const int it = kt0 + kspl;
+        const int kb = it * kKT;
+        if (it >= n_tiles || wave_rows == 0 || kb > wave_last_pos) continue;  // uniform
+        attend(kb, sKb[kspl], sVb[kspl]);
     }
 
     if constexpr (KSP > 1) {
@@ -688,7 +579,7 @@ prefill_mfma_kernel(PrefillParams p) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int m = 4 * lg + r;
-                    const int rot = vrot_of(m);
+                    const int rot = v_rot<NDT>(m);
 #pragma unroll
                     for (int c = 0; c < VC; ++c) {
                         float4 x;
@@ -724,13 +615,14 @@ hipError_t launch_t(const Shape& s, const PrefillParams& pp, hipStream_t st) {
     constexpr int QB = 16 * NQT * QS;
     const int n_qb = PAIR ? ((pp.n + 15) / 16 + 1) / 2 : (pp.n + QB - 1) / QB;
     const dim3 grid(n_qb * (s.num_heads / HW));
-    hipLaunchKernelGGL((prefill_mfma_kernel<HD, HW, QS, NQT, 32, 1, false, false, KSP, PAIR>),
+    hipLaunchKernelGGL((prefill_mfma_kernel<HD, HW, QS, NQT, KSP, PAIR>),
                        grid, dim3(64 * HW * QS * KSP), 0, st, pp);
     return hipGetLastError();
 }
 
 template <int HD>
 hipError_t launch_hd(const Shape& s, const PrefillParams& pp, hipStream_t st) {
+    // (at hd 128 only what prefill_split_plan() leaves comes here)
     switch (prefill_plan(s.head_dim, s.num_heads, s.kv_mul, s.cus, pp.start, pp.n)) {
         case PrefillKernel::kFourHeads: return launch_t<HD, 4, 1, 1>(s, pp, st);
         case PrefillKernel::kThreeHeads: return launch_t<HD, 3, 1, 1>(s, pp, st);
@@ -743,24 +635,9 @@ hipError_t launch_hd(const Shape& s, const PrefillParams& pp, hipStream_t st) {
             if constexpr (HD <= 96) return launch_t<HD, 4, 2, 1, true>(s, pp, st);
             break;
         case PrefillKernel::kDma:
-            if constexpr (HD == 128) {
-                const int n_qb = (pp.n + 31) / 32;
-                hipLaunchKernelGGL((prefill_mfma_kernel<128, 4, 2, 1, 32, 2, false, true>),
-                                   dim3(n_qb * (s.num_heads / 4)), dim3(512), 0, st, pp);
-                return hipGetLastError();
-            }
-            break;
         case PrefillKernel::kDmaPaired:
-            if constexpr (HD == 128) {
-                const int pwgs = ((pp.n + 15) / 16 + 1) / 2 * (s.num_heads / 4);
-                hipLaunchKernelGGL((prefill_mfma_kernel<128, 4, 2, 1, 32, 2, false, true, 1, true>),
-                                   dim3(pwgs), dim3(512), 0, st, pp);
-                return hipGetLastError();
-            }
-            break;
         case PrefillKernel::kPairedTwoHeads:
-            if constexpr (HD == 128) return launch_t<128, 2, 2, 2, true>(s, pp, st);
-            break;
+            break;  // hd 128: prefill_split_plan() takes these
         case PrefillKernel::kPairedOneHead:
             if constexpr (HD == 128) return launch_t<128, 1, 2, 4, true>(s, pp, st);
             break;
@@ -784,6 +661,9 @@ hipError_t launch_prefill_mfma(const Shape& s, const PrefillArgs& a, hipStream_t
                      a.n,   s.dim,     s.num_heads, s.kv_dim, s.kv_mul, s.half,
                      1.4426950408889634f / sqrtf((float)s.head_dim)};
     if (a.n > 65535 * 64) return hipErrorInvalidValue;
+    const PrefillSplit split =
+        prefill_split_plan(s.head_dim, s.num_heads, s.kv_mul, s.cus, a.start, a.n);
+    if (split != PrefillSplit::kNone) return launch_prefill_split(s, a, split, st);
     switch (s.head_dim) {
         case 16: return launch_hd<16>(s, pp, st);
         case 32: return launch_hd<32>(s, pp, st);

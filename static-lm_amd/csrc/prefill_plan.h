@@ -4,7 +4,10 @@
 
 namespace slm {
 
-// The prefill kernels, numbered as SLM_PF_* in slm_attn.h.
+// The tilings of a prefill, numbered as SLM_PF_* in slm_attn.h.  At hd 128
+// prefill_split_plan() below takes most batches to the split-bf16 kernel; its
+// rules name these tilings, and the measurements in prefill_plan() compare
+// the f32 kernels with each other.
 enum class PrefillKernel : int {
     kFourHeads = 0,
     kThreeHeads = 1,
@@ -129,6 +132,42 @@ inline PrefillKernel prefill_plan(int head_dim, int num_heads, int kv_mul, int c
     if (t.hw == 3) return PrefillKernel::kThreeHeads;
     if (t.hw == 2) return PrefillKernel::kTwoHeads;
     return PrefillKernel::kOneHead;
+}
+
+// Forms of the split-bf16 kernel (prefill_split.hip): eight waves per
+// workgroup, each one (head, 16-row block, key split).
+enum class PrefillSplit : int {
+    kNone = 0,         // the f32 kernel of prefill_plan()
+    kKeySplit = 1,     // four (head, block), paired blocks, two key splits
+    kPaired = 2,       // eight (head, block), paired blocks
+    kConsecutive = 3,  // eight (head, block), consecutive blocks
+};
+
+// Which batches run on bf16 matrix cores with split operands, and how: like
+// prefill_plan(), a pure function of the batch, the shape and the CU count.
+inline PrefillSplit prefill_split_plan(int head_dim, int num_heads, int kv_mul, int cus, int start,
+                                       int n) {
+    if (head_dim != 128) return PrefillSplit::kNone;
+    // Under four key tiles there is little to gain and the splitting's set-up
+    // shows (Llama-3-8B shape, per call, split against f32: 64 rows 13.6
+    // against 12.1 us, 128 rows 16.5 against 17.4).
+    if ((long)start + n < 128) return PrefillSplit::kNone;
+    // One head and four key splits per workgroup in f32 (135 KB of f32 tiles;
+    // four split tiles do not fit the LDS) stays ahead while it fits the CUs:
+    // 256 rows 20.7 against 22.1 us, 512 rows of 16 heads 28.4 against 32.9,
+    // 256 rows at start 8000 348 against 385.
+    if (prefill_plan(head_dim, num_heads, kv_mul, cus, start, n) == PrefillKernel::kPairedOneHead)
+        return PrefillSplit::kNone;
+    // All eight waves on as few columns as fill the CUs: with two key splits
+    // while that grid fits the CUs once (512 rows 34.3 against 39.5 us paired
+    // and 37.0 in f32; 512 rows at start 2000 131 against 181 and 180), then
+    // paired blocks while that does (1024 rows 71 against 91 and 87 us
+    // consecutive; 777 rows at start 1000 131 against 141), then consecutive
+    // ones (2048 rows 187 against 214 paired; 4096 rows 690 against 780).
+    const long cols = ((long)n + 15) / 16 * num_heads;
+    if (cols <= 4L * cus) return PrefillSplit::kKeySplit;
+    if (cols <= 8L * cus) return PrefillSplit::kPaired;
+    return PrefillSplit::kConsecutive;
 }
 
 }  // namespace slm

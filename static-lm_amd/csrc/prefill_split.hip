@@ -1,0 +1,588 @@
+// Causal prefill attention on bf16 matrix cores with f32 operands split in
+// three (v_mfma_f32_16x16x32_bf16) for gfx950.
+//
+// Replaces the per-row loop of forward_batch_with_kv (transformer.rs:563-593),
+// where row b at position p = start + b attends to cache rows 0..p.
+//
+// Precision.  An f32 value is the sum of three bf16 values x1 + x2 + x3 (each
+// the rounded remainder of the ones before), so a product is nine bf16
+// products, exact in f32; x2*y3, x3*y2 and x3*y3 (below 2^-25 of the product)
+// are left out.  The five small products and the leading one are summed
+// apart, and the output accumulators take one addition per 32-key tile, so
+// fewer roundings at full magnitude go into a result than with
+// v_mfma_f32_16x16x4_f32, which adds four products at a time.
+//
+// What bounds it: six bf16 products at 16 times the f32 MFMA rate.  A 16 x 32
+// x 128 product takes 48 MFMAs of 16 cycles against 64 of 32 for f32, and the
+// VALU work (softmax, splitting K, V and P) of one wave can run beside another
+// wave's MFMAs of a SIMD, which it cannot beside f32 MFMAs.
+//
+// Tiling.  A workgroup holds HW query heads of one KV head, two blocks of 16
+// query rows and KSP key splits, a wave for each; with PAIR the blocks are i
+// and n_blocks-1-i (every workgroup then has the same causal work), and the
+// waves are numbered key split first, then head, then block, so a SIMD holds
+// the same head and key split of the heavy and the light block.  Keys stream
+// through LDS in tiles of 32 rows (split k attends tiles k, k + KSP, ...),
+// split once per workgroup into three bf16 planes:
+//   S^T = K . Q^T    A = K rows, B = Q^T (registers): lane (lr = l%16, g =
+//                    l/16) ends with the scores of query lr against keys 16kk
+//                    + 4g + r in register r of subtile kk;
+//   O^T = V^T . P^T  A = V^T; B = P^T: lane group g supplies its own eight
+//                    probabilities, keys 4g + (0..3) and 16 + 4g + (0..3), so
+//                    they never move between lanes and V is stored with its
+//                    keys in that order.
+// Each wave's share of the next tiles goes from memory into its own LDS bytes
+// by DMA, so no registers are held for it.  With 80 KiB of LDS (KSP 1) two
+// workgroups share a CU, and one's MFMAs run beside the other's splitting.
+//
+// Non-finite values.  inf, and finite values that round to a bf16 inf, make
+// NaN when split.  A wave whose result is not finite therefore computes its
+// rows again in plain f32 from the cache (attend_plain).
+#include <math.h>
+
+#include "attn_common.h"
+#include "prefill_plan.h"
+#include "slm_internal.h"
+#include "tile_range.h"
+
+namespace slm {
+namespace {
+
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+struct SplitParams {
+    const float* q;
+    const float* k_cache;
+    const float* v_cache;
+    const float* cos_t;
+    const float* sin_t;
+    float* out;
+    int start;
+    int n;
+    int dim;
+    int num_heads;
+    int kv_dim;
+    int kv_mul;
+    int half;
+    float scale_log2;
+};
+
+__device__ __forceinline__ v4f mfma(bf8 a, bf8 b, v4f c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// Two values as bf16 pairs: x = p1 + p2 + p3 (24 bits).
+__device__ __forceinline__ void split2(float x0, float x1, uint32_t* p1, uint32_t* p2,
+                                       uint32_t* p3) {
+    const auto pack = [](float a, float b) {
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{a, b}, bf2));
+    };
+    *p1 = pack(x0, x1);
+    x0 -= __uint_as_float(*p1 << 16);
+    x1 -= __uint_as_float(*p1 & 0xFFFF0000u);
+    *p2 = pack(x0, x1);
+    x0 -= __uint_as_float(*p2 << 16);
+    x1 -= __uint_as_float(*p2 & 0xFFFF0000u);
+    *p3 = pack(x0, x1);
+}
+
+__device__ __forceinline__ void split8(const float (&x)[8], uint4 (&p)[3]) {
+    uint32_t w[3][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) split2(x[2 * i], x[2 * i + 1], &w[0][i], &w[1][i], &w[2][i]);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) p[k] = make_uint4(w[k][0], w[k][1], w[k][2], w[k][3]);
+}
+
+template <int HD, int HW, int QS, int KSP, bool PAIR>
+__global__ __launch_bounds__(64 * QS * HW * KSP, 2) void prefill_split_kernel(
+    SplitParams p) {
+    constexpr int NB = KSP == 1 ? 2 : 1;  // plane buffers
+    
+    constexpr int NWS = QS * HW;       // waves of one key split
+    constexpr int NW = NWS * KSP;
+    constexpr int NT = 64 * NW;
+    constexpr int KT = 32;             // keys per tile
+    constexpr int PL = KT * HD / 8;    // 16-byte chunks per plane of a K or V tile
+    constexpr int KC = HD / 8;         // chunks per K row
+    constexpr int NS = 2 * PL * KSP / NT;  // chunks a thread splits per step
+    constexpr int NKS = HD / 32;       // k-steps of K . Q^T
+    constexpr int NDT = HD / 16;       // 16-dim tiles of O^T
+    static_assert(2 * PL * KSP % NT == 0 && PL % 64 == 0, "whole chunks, a wave's in one tile");
+    static_assert(KC == 16, "k_slot");
+    // K planes: row r's chunk c (dims 8c..8c+7) in slot c ^ 2(r & 7).  V
+    // planes: dim d's chunk g (the keys lane group g supplies) in slot g ^
+    // v_swz(d).  A 64-lane ds_read_b128 is served in four cycles of 16 lanes of
+    // a half-wave that agree in the parity of lane bits 2-4 (bit 0 may also
+    // count); with these slots the 16 lanes of reads and stores cover the 64
+    // banks once, either way.
+    __shared__ __align__(16) struct {
+        uint4 k[NB * KSP][3][PL];
+        uint4 v[NB * KSP][3][PL];
+        float raw[2 * KSP * PL * 8];  // f32 K and V of the next step's tiles
+    } sm;
+    auto k_slot = [](int r, int c) { return r * KC + (c ^ ((r & 7) << 1)); };
+    auto v_swz = [](int d) { return ((d >> 4) & 1) | (((d >> 2) & 1) << 1); };
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 15;
+    const int lg = lane >> 4;
+    const int kspl = wave % KSP;
+    const int hw = wave / KSP % HW;
+    const int qs = wave / (KSP * HW);
+
+    // blockIdx.x = block pair * head groups + head group: consecutive
+    // workgroups go round-robin to the 8 XCDs, so with 8 head groups each XCD's
+    // L2 serves one KV head's K/V; longest causal ranges first.  With an odd
+    // block count the middle pair's second block is its first, and its waves
+    // hold no rows.
+    const int n_qb = (p.n + 15) / 16;
+    const int n_hg = p.num_heads / HW;
+    const int hg = (int)blockIdx.x % n_hg;
+    const int pi = (int)blockIdx.x / n_hg;
+    const int g = (hg * HW) / p.kv_mul;
+    const int head = hg * HW + hw;
+    int q0, last;  // first query row of this wave; the workgroup's rows end at last
+    if constexpr (PAIR) {
+        const int pj = pi * (QS / 2) + qs % (QS / 2);  // this wave's pair
+        const int heavy = n_qb - 1 - pj;
+        q0 = qs < QS / 2 ? (heavy >= pj ? heavy * 16 : p.n) : (pj < heavy ? pj * 16 : p.n);
+        last = min(p.n, (n_qb - pi * (QS / 2)) * 16);
+    } else {
+        const int qb = (n_qb + QS - 1) / QS - 1 - pi;
+        q0 = (qb * QS + qs) * 16;
+        last = min(p.n, (qb + 1) * QS * 16);
+    }
+    const int kv_len = p.start + last;
+    const int n_tiles = (kv_len + KT - 1) / KT;
+    const int wave_rows = max(0, min(16, p.n - q0));
+    const int wave_last_pos = p.start + q0 + wave_rows - 1;
+    const int row = q0 + lr;
+    const bool row_ok = row < p.n;
+
+    // dims 32 ks + 8 lg .. +7 of this lane's query, rotated and scaled
+    auto load_q8 = [&](int ks, float (&x)[8]) __attribute__((always_inline)) {
+        const long r = row_ok ? row : 0;
+        const float* src = p.q + r * p.dim + head * HD + 32 * ks + 8 * lg;
+        float4 a = ld4(src), b = ld4(src + 4);
+        if (p.cos_t) {
+            const long tr = (p.start + r) * (long)p.half + 16 * ks + 4 * lg;
+            const float4 c = ld4(p.cos_t + tr), s = ld4(p.sin_t + tr);
+            a = rope4_exact(a, make_float2(c.x, c.y), make_float2(s.x, s.y));
+            b = rope4_exact(b, make_float2(c.z, c.w), make_float2(s.z, s.w));
+        }
+        const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = row_ok ? v[i] * p.scale_log2 : 0.0f;
+    };
+
+    const float* kg = p.k_cache + g * HD;
+    const float* vg = p.v_cache + g * HD;
+    static_assert(tile_range_fits(KT, kMaxKvDim), "tile ranges must fit 32 bits");
+
+    // Shares.  A step's chunks are those of the KSP K tiles, then those of the
+    // V tiles; chunk i*NT + tid is this thread's, so a wave's 64 chunks lie in
+    // one tile.  Within it chunk f holds K row f / KC, dims 8 (f % KC) .., or
+    // V dim f % HD, lane group f / HD.  The wave's chunks arrive as two pieces
+    // of 64 16-byte loads (V piece h: keys 16h + 4g + (0..3) of the wave's 64
+    // dims), in raw bytes that only this wave reads back.
+    // (a step's tiles are whole multiples of the threads, or one tile is half)
+    auto share_v = [&](int i) {
+        return NT <= PL ? i * NT >= PL * KSP : i * NT + wave * 64 >= PL * KSP;
+    };
+    auto share_slot = [&](int i) {
+        return NT <= PL ? i * NT / PL % KSP : (i * NT + wave * 64) / PL % KSP;
+    };
+    auto share_first = [&](int i) { return (i * NT + wave * 64) % PL; };  // within the tile
+    int off[NS][2];
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+        const int fw = share_first(i);
+        const bool is_v = share_v(i);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int e = fw * 2 + h * 64 + lane;  // float4 of the tile
+            const int key = 16 * h + 4 * (fw / HD) + (lane >> 4);
+            off[i][h] = is_v ? (key * p.kv_dim + fw % HD + 4 * (lane & 15)) * 4
+                             : ((e / (HD / 4)) * p.kv_dim + (e % (HD / 4)) * 4) * 4;
+        }
+    }
+    // tiles kt0 .. kt0 + KSP - 1; those past the last read as zeros
+    auto dma = [&](int kt0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+            const int u = i * NT + wave * 64;  // uniform
+            const int kb = min(kt0 + share_slot(i), n_tiles) * KT;
+            const int bytes = kb < kv_len ? (int)tile_range_bytes(kv_len, kb, KT, p.kv_dim) : 0;
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<float*>((share_v(i) ? vg : kg) + (long)kb * p.kv_dim), 0, bytes,
+                0x00020000);
+            // inline assembly: the compiler must not make LDS reads of the
+            // planes wait for it; the wave waits (vmcnt) before it reads its
+            // share back.  M0 holds the wave's LDS destination; lane l's 16
+            // bytes land at M0 + 16*l.
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const unsigned dst = (unsigned)(unsigned long)(
+                    __attribute__((address_space(3))) float*)&sm.raw[u * 8 + h * 256];
+                asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off[i][h]), "s"(r),
+                             "{m0}"(dst) : "memory");
+            }
+        }
+    };
+    // Splits this wave's share into the planes of buffer buf.
+    auto stage = [&](int buf) __attribute__((always_inline)) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < NS; ++i) {
+            const int u = i * NT + wave * 64;
+            const int slot = buf * KSP + share_slot(i), f = share_first(i) + lane;
+            float x[8];
+            uint4 pl[3];
+            if (!share_v(i)) {  // uniform
+                const float4 a = ld4(&sm.raw[(u + lane) * 8]), b = ld4(&sm.raw[(u + lane) * 8 + 4]);
+                x[0] = a.x, x[1] = a.y, x[2] = a.z, x[3] = a.w;
+                x[4] = b.x, x[5] = b.y, x[6] = b.z, x[7] = b.w;
+                split8(x, pl);
+#pragma unroll
+                for (int k = 0; k < 3; ++k) sm.k[slot][k][k_slot(f / KC, f % KC)] = pl[k];
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) x[j] = sm.raw[u * 8 + j * 64 + lane];
+                split8(x, pl);
+                const int d = f % HD;
+#pragma unroll
+                for (int k = 0; k < 3; ++k) sm.v[slot][k][d * 4 + (f / HD ^ v_swz(d))] = pl[k];
+            }
+        }
+        // the raw bytes are read (and the planes written) before the next DMA
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    };
+
+    dma(0);
+    bf8 qf[3][NKS];  // Q^T fragments, three planes
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+        float x[8];
+        uint4 pl[3];
+        load_q8(ks, x);
+        split8(x, pl);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) qf[k][ks] = __builtin_bit_cast(bf8, pl[k]);
+    }
+
+    // Softmax state (log2 domain): m, the running max (-inf before the first
+    // key); om, the offset the score accumulators start from (negm holds -om:
+    // the K . Q^T MFMAs then return s - om, and exp2 takes them as they are);
+    // lim, how far a tile's max may exceed om before the state is rescaled
+    // (-inf before the first tile, which therefore always rescales).
+    v4f o[NDT], negm;
+    float m, l, om, lim;
+    auto reset = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NDT; ++i) o[i] = v4f{0.f, 0.f, 0.f, 0.f};
+        negm = v4f{0.f, 0.f, 0.f, 0.f};
+        m = -INFINITY;
+        l = 0.0f;
+        om = 0.0f;
+        lim = -INFINITY;
+    };
+    reset();
+
+    // Causal mask and online softmax of one tile: scores (less om) in,
+    // probabilities out.
+    auto softmax = [&](int kb, v4f (&s)[2]) __attribute__((always_inline)) {
+        if (kb + KT - 1 > p.start + q0) {  // uniform: some key may be masked
+            const int last_key = p.start + q0 + lr - kb - 4 * lg;
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (16 * kk + r > last_key) s[kk][r] = -INFINITY;
+        }
+        float mx = s[0][0];
+#pragma unroll
+        for (int j = 1; j < 8; ++j) mx = fmaxf(mx, s[j >> 2][j & 3]);
+        mx = rows_max(mx);
+        if (__any(mx > lim)) {  // wave-uniform
+            // without key splits the first tile holds key 0 <= qpos; with them
+            // it may mask every key of a query, whose state then stays empty
+            const float mn = fmaxf(m, mx + om);
+            const bool none = KSP > 1 && mn == -INFINITY;
+            const float alpha = none ? 1.0f : __builtin_amdgcn_exp2f(m - mn);
+            l *= alpha;
+#pragma unroll
+            for (int i = 0; i < NDT; ++i) o[i] *= alpha;
+            const float d = none ? 0.0f : mn - om;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) s[j >> 2][j & 3] -= d;
+            m = mn;
+            if (!none) {
+                om = mn;
+                lim = kLazyRescale;
+                negm = v4f{-mn, -mn, -mn, -mn};
+            }
+        }
+        float ps = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float e = __builtin_amdgcn_exp2f(s[j >> 2][j & 3]);
+            s[j >> 2][j & 3] = e;
+            ps = j == 0 ? e : ps + e;
+        }
+        l += ps;
+    };
+
+    // A tile from its planes.  The fragments come in groups of six, 12 MFMAs
+    // each; a group is read while the one before it is in use (two waves per
+    // SIMD do not cover the LDS latency by themselves).
+    auto attend = [&](int kb, int slot) __attribute__((always_inline)) {
+        constexpr int A[6] = {2, 0, 1, 1, 0, 0}, B[6] = {0, 2, 1, 0, 1, 0};
+        bf8 f[2][2][3];
+        auto load_k = [&](int ks, bf8 (&d)[2][3]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+                for (int k = 0; k < 3; ++k)
+                    d[kk][k] = __builtin_bit_cast(
+                        bf8, sm.k[slot][k][k_slot(16 * kk + lr, 4 * ks + lg)]);
+        };
+        auto load_v = [&](int dt, bf8 (&d)[2][3]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    const int dim = 16 * (dt + i) + lr;
+                    d[i][k] =
+                        __builtin_bit_cast(bf8, sm.v[slot][k][dim * 4 + (lg ^ v_swz(dim))]);
+                }
+        };
+        auto interleave = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < 6; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // an LDS read
+                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);  // two MFMAs
+            }
+        };
+        v4f s[2] = {negm, negm};
+        load_k(0, f[0]);
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) {
+            const bf8(&c)[2][3] = f[ks & 1];
+            if (ks + 1 < NKS)
+                load_k(ks + 1, f[(ks + 1) & 1]);
+            else
+                load_v(0, f[(ks + 1) & 1]);
+#pragma unroll
+            for (int e = 0; e < 6; ++e)
+#pragma unroll
+                for (int kk = 0; kk < 2; ++kk) s[kk] = mfma(c[kk][A[e]], qf[B[e]][ks], s[kk]);
+            interleave();
+        }
+        softmax(kb, s);
+        bf8 pf[3];
+        {
+            const float x[8] = {s[0][0], s[0][1], s[0][2], s[0][3],
+                                s[1][0], s[1][1], s[1][2], s[1][3]};
+            uint4 pl[3];
+            split8(x, pl);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) pf[k] = __builtin_bit_cast(bf8, pl[k]);
+        }
+#pragma unroll
+        for (int dt = 0; dt < NDT; dt += 2) {
+            const bf8(&c)[2][3] = f[(NKS + dt / 2) & 1];
+            if (dt + 2 < NDT) load_v(dt + 2, f[(NKS + dt / 2 + 1) & 1]);
+#pragma unroll
+            for (int e = 0; e < 6; ++e)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    o[dt + i] = mfma(c[i][A[e]], pf[B[e]], o[dt + i]);
+            interleave();
+        }
+    };
+
+    const int n_steps = (n_tiles + KSP - 1) / KSP;
+    if constexpr (NB == 1) {
+        for (int st = 0; st < n_steps; ++st) {
+            stage(0);
+            if (st + 1 < n_steps) dma((st + 1) * KSP);
+            __syncthreads();  // the planes are whole
+            const int kb = (st * KSP + kspl) * KT;
+            if (wave_rows > 0 && kb <= wave_last_pos) attend(kb, kspl);  // wave-uniform
+            __syncthreads();  // every wave is done with them
+        }
+    } else {
+        // Half of a SIMD's waves split the next tile before they attend this
+        // one, the others afterwards, so that splitting runs beside MFMAs.
+        auto next = [&](int st, int buf) __attribute__((always_inline)) {
+            if (st + 1 >= n_steps) return;
+            stage(buf ^ 1);
+            if (st + 2 < n_steps) dma(st + 2);
+        };
+        stage(0);
+        if (n_steps > 1) dma(1);
+        for (int st = 0; st < n_steps; ++st) {
+            // the planes of tile st are whole, and every wave is done with the
+            // other buffer
+            __syncthreads();
+            const int buf = st & 1;
+            if (qs & 1) next(st, buf);
+            const int kb = st * KT;
+            if (wave_rows > 0 && kb <= wave_last_pos) attend(kb, buf);  // wave-uniform
+            if (!(qs & 1)) next(st, buf);
+        }
+    }
+
+    if constexpr (KSP > 1) {
+        // Merge of the key splits: splits 1..KSP-1 hand each lane's O
+        // registers, max and sum partial to split 0 through LDS (lane
+        // contiguous), which folds them in split order.
+        constexpr int NR = NDT * 4 + 2;  // floats per lane
+        static_assert((KSP - 1) * NWS * 64 * NR * 4 <= (int)sizeof(sm), "the merge fits the LDS");
+        float* s_merge = reinterpret_cast<float*>(&sm);
+        const int ws = qs * HW + hw;
+        if (kspl > 0) {
+            float* dst = s_merge + ((kspl - 1) * NWS + ws) * NR * 64 + lane;
+#pragma unroll
+            for (int i = 0; i < NDT; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) dst[64 * (4 * i + r)] = o[i][r];
+            dst[64 * (NR - 2)] = m;
+            dst[64 * (NR - 1)] = l;
+        }
+        __syncthreads();
+        if (kspl > 0) return;  // no barrier follows
+        float mk[KSP];
+        float mx = m;
+#pragma unroll
+        for (int k = 1; k < KSP; ++k) {
+            mk[k] = s_merge[((k - 1) * NWS + ws) * NR * 64 + lane + 64 * (NR - 2)];
+            mx = fmaxf(mx, mk[k]);
+        }
+        const float s0 = __builtin_amdgcn_exp2f(m - mx);
+        l *= s0;
+#pragma unroll
+        for (int i = 0; i < NDT; ++i) o[i] *= s0;
+#pragma unroll
+        for (int k = 1; k < KSP; ++k) {
+            const float* src = s_merge + ((k - 1) * NWS + ws) * NR * 64 + lane;
+            const float sk = __builtin_amdgcn_exp2f(mk[k] - mx);
+            l += src[64 * (NR - 1)] * sk;
+#pragma unroll
+            for (int i = 0; i < NDT; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[i][r] += src[64 * (4 * i + r)] * sk;
+        }
+    }
+
+    if (wave_rows == 0) return;
+    // A tile in f32 arithmetic from the cache rows; masked keys take no part
+    // in the sums.
+    auto attend_plain = [&](int kb) __attribute__((always_inline)) {
+        v4f s[2];
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) s[kk] = v4f{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+#pragma unroll 1
+        for (int k = 0; k < KT && kb + k < kv_len; ++k) {
+            const float* kr = kg + (long)(kb + k) * p.kv_dim + 8 * lg;
+            float d = 0.0f;
+#pragma unroll 1
+            for (int ks = 0; ks < NKS; ++ks) {
+                float x[8];
+                load_q8(ks, x);
+                const float4 a = ld4(kr + 32 * ks), b = ld4(kr + 32 * ks + 4);
+                const float y[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+                for (int i = 0; i < 8; ++i) d = fmaf(x[i], y[i], d);
+            }
+            d += __shfl_xor(d, 16);
+            d += __shfl_xor(d, 32);
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (16 * (j >> 2) + 4 * lg + (j & 3) == k) s[j >> 2][j & 3] = d - om;
+        }
+        softmax(kb, s);
+#pragma unroll 1
+        for (int k = 0; k < KT && kb + k < kv_len; ++k) {
+            float pk = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (16 * (j >> 2) + 4 * lg + (j & 3) == k) pk = s[j >> 2][j & 3];
+            pk = __shfl(pk, lr + 16 * ((k >> 2) & 3));
+            const bool on = kb + k <= p.start + row;
+            const float* vr = vg + (long)(kb + k) * p.kv_dim + 4 * lg;
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt) {
+                const float4 v = ld4(vr + 16 * dt);
+                const float w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (on) o[dt][r] = fmaf(w[r], pk, o[dt][r]);
+            }
+        }
+    };
+    float lt = rows_sum(l);
+    float z = lt * 0.0f;  // NaN once any of the row's values is not finite
+#pragma unroll
+    for (int i = 0; i < NDT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) z = fmaf(o[i][r], 0.0f, z);
+    if (__any(row_ok && z != z)) {
+        reset();
+#pragma unroll 1
+        for (int kb = 0; kb <= wave_last_pos; kb += KT) attend_plain(kb);
+        lt = rows_sum(l);
+    }
+
+    // normalise and store: lane holds out[row][16 dt + 4 lg + (0..3)]
+    if (row_ok) {
+        const float inv = 1.0f / lt;
+        float* dst = p.out + (long)row * p.dim + head * HD + 4 * lg;
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt)
+            *reinterpret_cast<float4*>(dst + 16 * dt) =
+                make_float4(o[dt][0] * inv, o[dt][1] * inv, o[dt][2] * inv, o[dt][3] * inv);
+    }
+}
+
+template <int HW, int QS, int KSP, bool PAIR>
+hipError_t launch_t(const Shape& s, const SplitParams& pp, hipStream_t st) {
+    const int groups = ((pp.n + 15) / 16 + QS - 1) / QS;
+    hipLaunchKernelGGL((prefill_split_kernel<128, HW, QS, KSP, PAIR>),
+                       dim3(groups * (s.num_heads / HW)), dim3(64 * QS * HW * KSP), 0, st, pp);
+    return hipGetLastError();
+}
+
+template <int HW>
+hipError_t launch_hw(const Shape& s, const SplitParams& pp, PrefillSplit form, hipStream_t st) {
+    switch (form) {
+        case PrefillSplit::kKeySplit: return launch_t<HW, 4 / HW, 2, true>(s, pp, st);
+        case PrefillSplit::kPaired: return launch_t<HW, 8 / HW, 1, true>(s, pp, st);
+        case PrefillSplit::kConsecutive: return launch_t<HW, 8 / HW, 1, false>(s, pp, st);
+        case PrefillSplit::kNone: break;
+    }
+    return hipErrorInvalidValue;
+}
+
+}  // namespace
+
+hipError_t launch_prefill_split(const Shape& s, const PrefillArgs& a, PrefillSplit form,
+                                hipStream_t st) {
+    SplitParams pp{a.q,   a.k_cache, a.v_cache,   a.cos_t,  a.sin_t,  a.out, a.start,
+                   a.n,   s.dim,     s.num_heads, s.kv_dim, s.kv_mul, s.half,
+                   1.4426950408889634f / sqrtf((float)s.head_dim)};
+    if (s.head_dim != 128) return hipErrorInvalidValue;
+    // four heads on the tiles where there are so many: 4096 rows of the
+    // Llama-3-8B shape 672 against 690 us with two
+    if (form == PrefillSplit::kConsecutive && s.kv_mul % 4 == 0)
+        return launch_t<4, 2, 1, false>(s, pp, st);
+    return s.kv_mul % 2 == 0 ? launch_hw<2>(s, pp, form, st) : launch_hw<1>(s, pp, form, st);
+}
+
+}  // namespace slm

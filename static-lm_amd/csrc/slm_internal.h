@@ -69,8 +69,8 @@ hipError_t launch_decode(const Shape& s, const DecodeArgs& a, hipStream_t st);
 // Merge of the split partials; needed only when a.n_splits > 1.
 hipError_t launch_decode_combine(const Shape& s, const DecodeArgs& a, hipStream_t st);
 
-// Causal prefill on fp32 MFMA: rows b < n at positions start + b attend to
-// cache rows 0..start+b.  q is un-rotated when cos_t != nullptr.
+// Causal prefill on the matrix cores: rows b < n at positions start + b
+// attend to cache rows 0..start+b.  q is un-rotated when cos_t != nullptr.
 struct PrefillArgs {
     const float* q;
     const float* k_cache;
@@ -83,6 +83,12 @@ struct PrefillArgs {
 };
 hipError_t launch_prefill_mfma(const Shape& s, const PrefillArgs& a,
                                hipStream_t st);
+// The same on bf16 matrix cores with f32 operands split in three
+// (prefill_split.hip), in the form that prefill_split_plan() gives;
+// launch_prefill_mfma calls it.
+enum class PrefillSplit : int;
+hipError_t launch_prefill_split(const Shape& s, const PrefillArgs& a, PrefillSplit form,
+                                hipStream_t st);
 
 // Q4_0 x Q8_0 projections (quant_gemm.hip).  A job is one weight matrix:
 // nibbles [rows][nb][16], f16 scales [rows][q4_scale_stride(nb)],

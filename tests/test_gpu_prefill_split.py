@@ -1,0 +1,110 @@
+"""The split-bf16 prefill (head_dim 128) at the sizes where its forms, blocks
+and key tiles begin and end, against float64 attention, and with values that
+cannot be split."""
+import numpy as np
+import pytest
+
+from slm_testlib import gen, load_product
+
+P = load_product()
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+HD = 128
+
+
+def run(heads, kvh, start, q, k, v):
+    """attend_batch of rotated q [n][heads*HD] over cache rows 0..start+n-1."""
+    rows, n = k.shape[0], q.shape[0]
+    with P.AttentionContext(heads * HD, heads, kvh, max(rows, 16), 1) as ctx:
+        ctx.kv_write(0, 0, 0, k)
+        ctx.kv_write(0, 1, 0, v)
+        qd = torch.from_numpy(q).cuda()
+        out = torch.full_like(qd, float("nan"))
+        torch.cuda.synchronize()
+        ctx.attend_batch_dev(0, start, n, qd.data_ptr(), out.data_ptr())
+        ctx.sync()
+        return out.cpu().numpy()
+
+
+def attend64(heads, kvh, start, q, k, v):
+    """float64 attention; (out, per-element sum of |p v|, largest |score|)."""
+    n = q.shape[0]
+    out, mag, smax = np.empty(q.shape), np.empty(q.shape), 0.0
+    mask = np.arange(k.shape[0])[None, :] > start + np.arange(n)[:, None]
+    for h in range(heads):
+        g = h // (heads // kvh)
+        hs, gs = slice(h * HD, (h + 1) * HD), slice(g * HD, (g + 1) * HD)
+        s = q[:, hs].astype(np.float64) @ k[:, gs].astype(np.float64).T / np.sqrt(HD)
+        s[mask] = -np.inf
+        smax = max(smax, np.abs(s[~mask]).max())
+        p = np.exp(s - s.max(1, keepdims=True))
+        p /= p.sum(1, keepdims=True)
+        out[:, hs] = p @ v[:, gs].astype(np.float64)
+        mag[:, hs] = p @ np.abs(v[:, gs].astype(np.float64))
+    return out, mag, smax
+
+
+# heads, kv_heads, start, n: one, two, three, four and eight heads per KV head;
+# key splits, paired and consecutive blocks; block and tile edges (15/16/17
+# rows, 127 to 129 and 159 to 161 keys), odd and even block counts
+CASES = [
+    (2, 1, 112, 16), (2, 1, 111, 17), (2, 1, 113, 15), (4, 1, 0, 128), (4, 1, 0, 129),
+    (1, 1, 100, 28), (1, 1, 127, 33), (3, 1, 0, 160), (3, 3, 30, 131), (8, 1, 96, 65),
+    (12, 4, 0, 250), (2, 2, 1000, 2), (4, 2, 500, 47),
+    (32, 8, 0, 545), (32, 32, 3, 528), (32, 8, 0, 1025), (24, 8, 40, 1400), (32, 16, 0, 1040),
+]
+
+
+@pytest.mark.parametrize("heads,kvh,start,n", CASES)
+def test_against_float64(heads, kvh, start, n):
+    rows = start + n
+    q = gen([71, heads, start, n], (n, heads * HD)) * np.float32(4)
+    k = gen([72, heads, start, n], (rows, kvh * HD)) * np.float32(2)
+    v = gen([73, heads, start, n], (rows, kvh * HD))
+    ref, mag, smax = attend64(heads, kvh, start, q, k, v)
+    got = run(heads, kvh, start, q, k, v)
+    # Roundings of 2^-24: six per 32-key tile in an output sum and one in the
+    # row sum, per score 24 accumulations (of partial sums taken as at most
+    # twice the largest score, in log2 units) and the pre-scaled q, and a few
+    # in exp2, the normalisation and the dropped products.
+    tiles = (rows + 31) // 32
+    bound = (7 * tiles + 2 * 25 * 1.4427 * smax + 16) * 2.0 ** -24
+    err = np.abs(got - ref) / mag
+    assert err.max() <= bound, (err.max(), bound)
+    # and on average far below: the roundings are not all one way
+    rel = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    assert rel < 3e-6, rel
+
+
+@pytest.mark.parametrize("heads,kvh,start,n", [(2, 1, 100, 60), (32, 8, 0, 600), (32, 32, 0, 1100)])
+def test_values_that_cannot_be_split(heads, kvh, start, n):
+    """-inf scores drop their key, inf and near-overflow values travel, and
+    earlier rows and other KV heads do not see them."""
+    rows = start + n
+    q = np.abs(gen([74, n], (n, heads * HD))) + np.float32(0.1)
+    k = gen([75, n], (rows, kvh * HD))
+    v = gen([76, n], (rows, kvh * HD))
+    j_k, j_v, j_big = rows - 45, rows - 20, rows - 9
+    # its probability stays small beside a running max that may lag by 2^8
+    k[j_big, :HD] = -2
+    k2, v2 = k.copy(), v.copy()
+    k2[j_k, :HD] = -np.inf           # every score of KV head 0 there is -inf
+    v2[j_v, 3] = np.inf
+    v2[j_big, 5] = np.float32(3.4e38)  # rounds to a bf16 infinity
+    got = run(heads, kvh, start, q, k2, v2)
+    kr = k.copy()
+    kr[j_k, :HD] = np.float32(-1e4)  # exp underflows to 0: the key drops out
+    vr = v.copy()
+    vr[j_v, 3] = 0
+    vr[j_big, 5] = 0
+    ref, mag, _ = attend64(heads, kvh, start, q, kr, vr)
+    pos = start + np.arange(n)
+    per = heads // kvh
+    cols0 = np.arange(per) * HD      # KV head 0's query heads
+    assert np.isposinf(got[np.ix_(pos >= j_v, cols0 + 3)]).all()
+    big = got[np.ix_(pos >= j_big, cols0 + 5)]
+    assert np.isfinite(big).all() and (big > 1e30).all()
+    ok = np.ones(got.shape, bool)
+    ok[np.ix_(pos >= j_v, cols0 + 3)] = False
+    ok[np.ix_(pos >= j_big, cols0 + 5)] = False
+    assert (np.abs(got - ref)[ok] <= 2e-5 * np.maximum(mag, 1e-3)[ok]).all()
