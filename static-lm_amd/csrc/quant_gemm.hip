@@ -27,6 +27,8 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "attn_common.h"
 #include "jit_math.h"
 #include "norm_common.h"
@@ -966,6 +968,143 @@ __global__ __launch_bounds__(64 * WRW * WTW) void gemm_q4_mfma_kernel(GemmParams
 #undef SLM_GEMM_LOAD_STAGE
 #undef SLM_GEMM_STORE_STAGE
 
+// ---- MFMA GEMM of few outputs: the blocks split over the waves ----
+//
+// A product with few tiles is bound by the tile's walk along its row: one
+// stage of blocks after another, a memory round trip each.  Here a workgroup
+// takes 16 rows x 16 tokens, and its eight waves take four blocks each of
+// every 32.  Lane (lr = l%16, g = l/16) loads block g of the four whole, for
+// row and token lr (one 16-byte load of weights, two of activations, with no
+// line fetched in pieces); a transpose over the lane groups then gives it
+// elements 4g..4g+3 and 16+4g..16+4g+3 of each block, the K order of both
+// operands of v_mfma_i32_16x16x32_i8.  It ends with tokens 4g..4g+3 of row lr,
+// whose terms (float(D) * (dw*da)) it leaves in LDS.  The scalar dot's one
+// ordered f32 sum per output is then taken by a thread each, 32 terms at a
+// time, while the other waves compute the next 32 blocks' terms.
+constexpr int kSmallWaves = 8;
+constexpr int kSmallBlocks = 4;  // blocks per wave and chunk
+constexpr int kSmallChunk = kSmallWaves * kSmallBlocks;
+constexpr int kSmallRows = 16, kSmallToks = 16;
+
+__global__ __launch_bounds__(64 * kSmallWaves, 4) void gemm_q4_small_kernel(GemmParams p) {
+#pragma clang fp contract(off)
+    __shared__ __align__(16) float s_t[2][kSmallChunk][kSmallToks * kSmallRows];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 15;
+    const int lg = lane >> 4;
+    const int n_tt = (p.batch + kSmallToks - 1) / kSmallToks;
+    int rt = blockIdx.x / n_tt;
+    const int tt = blockIdx.x - rt * n_tt;
+    int m = 0;
+    while (m < p.nmat - 1 && rt >= p.tiles[m]) {
+        rt -= p.tiles[m];
+        ++m;
+    }
+    const QMat M = pick(p.m, m);
+    const int nb = p.nb;
+    const int ds = p.d_stride;
+    const int wr0 = rt * kSmallRows, wt0 = tt * kSmallToks;
+
+    // addresses clamped into the buffers: rows, tokens and blocks past the end
+    // are never used
+    const long row = min(wr0 + lr, M.rows - 1);
+    const uint8_t* asrc = M.qs + row * nb * 16;
+    const uint16_t* dwsrc = M.d + row * ds;
+    const uint32_t* bsrc = p.aq + (long)min(wt0 + lr, p.batch - 1) * nb * 8;
+    const float* dasrc[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) dasrc[r] = p.ad + (long)min(wt0 + 4 * lg + r, p.batch - 1) * ds;
+
+    struct Loads {
+        uint4 w, b0, b1;
+        uint2 dw;
+        float4 da[4];
+    };
+    auto load = [&](int c, Loads& L) __attribute__((always_inline)) {
+        const int b0 = c * kSmallChunk + wave * kSmallBlocks;
+        const int b = min(b0 + lg, nb - 1);
+        L.w = *reinterpret_cast<const uint4*>(asrc + (long)b * 16);
+        L.b0 = *reinterpret_cast<const uint4*>(bsrc + (long)b * 8);
+        L.b1 = *reinterpret_cast<const uint4*>(bsrc + (long)b * 8 + 4);
+        const int s0 = min(b0, ds - kSmallBlocks);  // rows of scales hold ds >= 8
+        L.dw = *reinterpret_cast<const uint2*>(dwsrc + s0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) L.da[r] = ld4(dasrc[r] + s0);
+    };
+    // x[j] of lane group g becomes x[g] of lane group j
+    auto transpose = [](uint4 v, uint32_t (&x)[4]) __attribute__((always_inline)) {
+        const auto a = __builtin_amdgcn_permlane32_swap(v.x, v.z, false, false);
+        const auto b = __builtin_amdgcn_permlane32_swap(v.y, v.w, false, false);
+        const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+        const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+        x[0] = c[0], x[1] = c[1], x[2] = d[0], x[3] = d[1];
+    };
+    auto terms = [&](const Loads& L, int buf) __attribute__((always_inline)) {
+        uint32_t w[4], x0[4], x1[4];
+        transpose(L.w, w);
+        transpose(L.b0, x0);
+        transpose(L.b1, x1);
+#pragma unroll
+        for (int i = 0; i < kSmallBlocks; ++i) {
+            const uint32_t w0 = nib_to_i8(w[i] & 0x0F0F0F0Fu);
+            const uint32_t w1 = nib_to_i8((w[i] >> 4) & 0x0F0F0F0Fu);
+            const v4i d = __builtin_amdgcn_mfma_i32_16x16x32_i8(
+                (long)(((uint64_t)x1[i] << 32) | x0[i]), (long)(((uint64_t)w1 << 32) | w0),
+                v4i{0, 0, 0, 0}, 0, 0, 0);
+            const uint32_t dw2 = i < 2 ? L.dw.x : L.dw.y;
+            const float dw = h2f((uint16_t)(i & 1 ? dw2 >> 16 : dw2 & 0xFFFF));
+            float t[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float4 a = L.da[r];
+                const float sc = dw * (i == 0 ? a.x : i == 1 ? a.y : i == 2 ? a.z : a.w);
+                t[r] = (float)d[r] * sc;
+            }
+            *reinterpret_cast<float4*>(
+                &s_t[buf][wave * kSmallBlocks + i][lr * kSmallToks + 4 * lg]) =
+                make_float4(t[0], t[1], t[2], t[3]);
+        }
+    };
+    float acc = 0.0f;  // output tid (threads 0..255): row tid / 16, token tid % 16
+    auto sum = [&](int c, int buf) __attribute__((always_inline)) {
+        if (wave >= 4) return;
+        const int left = nb - c * kSmallChunk;
+        if (left >= kSmallChunk) {
+#pragma unroll
+            for (int b = 0; b < kSmallChunk; ++b) acc = acc + s_t[buf][b][tid];
+        } else {
+            for (int b = 0; b < left; ++b) acc = acc + s_t[buf][b][tid];
+        }
+    };
+
+    const int n_chunks = (nb + kSmallChunk - 1) / kSmallChunk;
+    Loads L[2];
+    load(0, L[0]);
+    auto step = [&](int c, auto buf_c) __attribute__((always_inline)) {
+        constexpr int buf = decltype(buf_c)::value;
+        if (c + 1 < n_chunks) load(c + 1, L[buf ^ 1]);
+        terms(L[buf], buf);
+        // the chunk's terms are whole; the sums over the other buffer ended
+        // before this barrier
+        __syncthreads();
+        sum(c, buf);
+    };
+    for (int c = 0; c < n_chunks; c += 2) {
+        step(c, std::integral_constant<int, 0>());
+        if (c + 1 < n_chunks) step(c + 1, std::integral_constant<int, 1>());
+    }
+
+    if (tid < kSmallToks * kSmallRows) {
+        const int t = wt0 + tid % kSmallToks, r = wr0 + tid / kSmallToks;
+        if (t < p.batch && r < M.rows) {
+            const long o = (long)t * M.out_stride + r;
+            M.out[o] = M.res ? M.res[o] + acc : acc;
+        }
+    }
+}
+
 size_t gemv_lds_bytes(int nt, int nb) {
     return ((size_t)gemv_terms_offset(nt, nb) + (size_t)nt * kGemvRows * kTermStride) * 4;
 }
@@ -1131,16 +1270,15 @@ hipError_t launch_swiglu_any(const Q4Job& gate, const Q4Job& up, const GemvAct& 
     }
 }
 
-template <int WRW, int WTW, int NTS>
-hipError_t launch_gemm_t(const Q4Job* jobs, int njobs, const uint32_t* aq, const float* ad,
-                         int nb, int batch, hipStream_t st) {
-    using Sh = GemmShape<WRW, WTW, NTS>;
+// The kernel's parameters and its grid of rt x tt tiles (0: too many).
+unsigned gemm_params(const Q4Job* jobs, int njobs, const uint32_t* aq, const float* ad, int nb,
+                     int batch, int rt, int tt, GemmParams* out) {
     GemmParams p{};
     long tiles = 0;
     for (int i = 0; i < njobs; ++i) {
         p.m[i] = QMat{jobs[i].qs, jobs[i].d, jobs[i].out, jobs[i].res, jobs[i].rows,
                       jobs[i].out_stride, q4_scale_stride(nb)};
-        p.tiles[i] = (jobs[i].rows + Sh::RT - 1) / Sh::RT;
+        p.tiles[i] = (jobs[i].rows + rt - 1) / rt;
         tiles += p.tiles[i];
     }
     p.nmat = njobs;
@@ -1149,10 +1287,29 @@ hipError_t launch_gemm_t(const Q4Job* jobs, int njobs, const uint32_t* aq, const
     p.nb = nb;
     p.d_stride = q4_scale_stride(nb);
     p.batch = batch;
-    const long n_tt = (batch + Sh::TT - 1) / Sh::TT;
-    if (tiles * n_tt > 0x7FFFFFFF) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((gemm_q4_mfma_kernel<WRW, WTW, NTS>), dim3((unsigned)(tiles * n_tt)),
-                       dim3(Sh::NT), 0, st, p);
+    *out = p;
+    const long grid = tiles * ((batch + tt - 1) / tt);
+    return grid > 0x7FFFFFFF ? 0 : (unsigned)grid;
+}
+
+template <int WRW, int WTW, int NTS>
+hipError_t launch_gemm_t(const Q4Job* jobs, int njobs, const uint32_t* aq, const float* ad,
+                         int nb, int batch, hipStream_t st) {
+    using Sh = GemmShape<WRW, WTW, NTS>;
+    GemmParams p;
+    const unsigned grid = gemm_params(jobs, njobs, aq, ad, nb, batch, Sh::RT, Sh::TT, &p);
+    if (!grid) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((gemm_q4_mfma_kernel<WRW, WTW, NTS>), dim3(grid), dim3(Sh::NT), 0, st, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_gemm_small(const Q4Job* jobs, int njobs, const uint32_t* aq, const float* ad,
+                             int nb, int batch, hipStream_t st) {
+    GemmParams p;
+    const unsigned grid =
+        gemm_params(jobs, njobs, aq, ad, nb, batch, kSmallRows, kSmallToks, &p);
+    if (!grid) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(gemm_q4_small_kernel, dim3(grid), dim3(64 * kSmallWaves), 0, st, p);
     return hipGetLastError();
 }
 
@@ -1230,7 +1387,17 @@ long device_cus() {
 
 }  // namespace
 
-// Tile choice: 128 x 128 workgroups (one per CU; 10% less VALU per output
+// Tile choice.  Up to four 16 x 16 workgroups per CU the blocks are split over
+// the waves (gemm_q4_small_kernel): its time grows with the workgroups (25 ns
+// each at 128 blocks, beside a floor of about 8 us), that of the tiles below
+// with the row's length only.  Per call with the quantization, tiles against
+// split: 4096 x 4096, 12 / 32 / 64 / 128 tokens (256 / 512 / 1024 / 2048
+// workgroups) 35 / 35 / 36 / 37 against 11 / 17 / 28 / 48 us; 4096 x 14336, 16 / 64
+// tokens 111 / 113 against 29 / 80; 14336 x 4096, 16 / 32 tokens (896 / 1792) 35.7 /
+// 36.2 against 27 / 43; 576 x 1536, 130 / 512 tokens (324 / 1152) 17.2 / 17.8 against
+// 10.1 / 18.7.
+//
+// Otherwise 128 x 128 workgroups (one per CU; 10% less VALU per output
 // element and block, measured on the 4096-token Q/K/V GEMM: 0.48 against
 // 0.53 ms) or 64 x 64 (two per CU).  The estimate of each is the workgroups
 // a CU runs in turn times one workgroup's work; products with few big tiles
@@ -1240,14 +1407,17 @@ long device_cus() {
 hipError_t launch_q4_gemm(const Q4Job* jobs, int njobs, const uint32_t* aq, const float* ad,
                           int nb, int batch, hipStream_t st) {
     if (njobs < 1 || njobs > 3 || batch < 1) return hipErrorInvalidValue;
-    long w128 = 0, w64 = 0;
+    long w128 = 0, w64 = 0, w16 = 0;
     for (int i = 0; i < njobs; ++i) {
         w128 += (long)((jobs[i].rows + 127) / 128) * ((batch + 127) / 128);
         w64 += (long)((jobs[i].rows + 63) / 64) * ((batch + 63) / 64);
+        w16 += (long)((jobs[i].rows + kSmallRows - 1) / kSmallRows) *
+               ((batch + kSmallToks - 1) / kSmallToks);
     }
     const long cus = device_cus();
     const double t128 = (double)((w128 + cus - 1) / cus) * 4.0;
     const double t64 = (double)((w64 + cus - 1) / cus) * 1.1;
+    if (w16 <= 4 * cus) return launch_gemm_small(jobs, njobs, aq, ad, nb, batch, st);
     return t128 < t64 ? launch_gemm_t<4, 2, 4>(jobs, njobs, aq, ad, nb, batch, st)
                       : launch_gemm_t<2, 2, 2>(jobs, njobs, aq, ad, nb, batch, st);
 }
