@@ -245,10 +245,10 @@ int slm_attn_decode_splits(const slm_attn_ctx* ctx, int32_t seq_len,
  * and benchmarks that need to know which batches run alike.  Heads per
  * workgroup are query heads of one KV head; query blocks are 16 rows;
  * "paired" workgroups take blocks i and n_blocks-1-i, so every workgroup has
- * the same causal work.  With head_dim 128 every tiling but the paired one
- * head one runs on bf16 matrix cores with f32 operands split in three, eight
- * waves of one head and block per workgroup, once start + n reaches 128 rows;
- * the others run on f32 ones as named.  SLM_ERR_BATCH as slm_attn_prefill for
+ * the same causal work.  The tilings are those of the f32 matrix kernels; most
+ * larger batches of head_dim 64 and 128 run instead on bf16 matrix cores with
+ * f32 operands split in three, eight waves of one head and block (or half a
+ * block's keys) per workgroup.  SLM_ERR_BATCH as slm_attn_prefill for
  * an empty or out-of-range batch. */
 enum {
     SLM_PF_FOUR_HEADS = 0,        /* four heads, one block (kv_mul % 4 == 0) */

@@ -4,9 +4,9 @@
 
 namespace slm {
 
-// The tilings of a prefill, numbered as SLM_PF_* in slm_attn.h.  At hd 128
-// prefill_split_plan() below takes most batches to the split-bf16 kernel; its
-// rules name these tilings, and the measurements in prefill_plan() compare
+// The tilings of a prefill, numbered as SLM_PF_* in slm_attn.h.  At hd 64 and
+// 128 prefill_split_plan() below takes most larger batches to the split-bf16
+// kernel, and the measurements in prefill_plan() compare
 // the f32 kernels with each other.
 enum class PrefillKernel : int {
     kFourHeads = 0,
@@ -147,6 +147,23 @@ enum class PrefillSplit : int {
 // prefill_plan(), a pure function of the batch, the shape and the CU count.
 inline PrefillSplit prefill_split_plan(int head_dim, int num_heads, int kv_mul, int cus, int start,
                                        int n) {
+    const long cols = ((long)n + 15) / 16 * num_heads;  // (head, 16-row block)
+    if (head_dim == 64) {
+        // Half the arithmetic per key tile of hd 128 behind the same set-up
+        // and barriers, so it takes more columns to win, and the f32 kernel's
+        // four key splits serve what does not fill the CUs: from three
+        // columns per CU (32 heads in 8 KV heads: 256 rows, two per CU, 13.8
+        // against 12.5 us in f32, 384 rows 17.6 against 20.8, 512 rows 20.8
+        // against 26.7; 9 in 3: 2048 rows, 4.5 per CU, 68.3 against 67.4).  Key
+        // splits up to eight columns per CU (16 heads, 2048 rows: 79.7 us,
+        // paired 81.4, f32 109.9; 3000 rows: 152, 139, 201), paired blocks up
+        // to sixteen (32 heads, 2048 rows: 106 us, consecutive 112, f32 150;
+        // 3000 rows: 214, 200, 312).
+        if (cols < 3L * cus) return PrefillSplit::kNone;
+        return cols <= 8L * cus    ? PrefillSplit::kKeySplit
+               : cols <= 16L * cus ? PrefillSplit::kPaired
+                                   : PrefillSplit::kConsecutive;
+    }
     if (head_dim != 128) return PrefillSplit::kNone;
     // Under four key tiles there is little to gain and the splitting's set-up
     // shows (Llama-3-8B shape, per call, split against f32: 64 rows 13.6
@@ -164,7 +181,6 @@ inline PrefillSplit prefill_split_plan(int head_dim, int num_heads, int kv_mul, 
     // paired blocks while that does (1024 rows 71 against 91 and 87 us
     // consecutive; 777 rows at start 1000 131 against 141), then consecutive
     // ones (2048 rows 187 against 214 paired; 4096 rows 690 against 780).
-    const long cols = ((long)n + 15) / 16 * num_heads;
     if (cols <= 4L * cus) return PrefillSplit::kKeySplit;
     if (cols <= 8L * cus) return PrefillSplit::kPaired;
     return PrefillSplit::kConsecutive;

@@ -112,8 +112,9 @@ __global__ __launch_bounds__(64 * QS * HW * KSP, 2) void prefill_split_kernel(
     constexpr int NKS = HD / 32;       // k-steps of K . Q^T
     constexpr int NDT = HD / 16;       // 16-dim tiles of O^T
     static_assert(2 * PL * KSP % NT == 0 && PL % 64 == 0, "whole chunks, a wave's in one tile");
-    static_assert(KC == 16, "k_slot");
-    // K planes: row r's chunk c (dims 8c..8c+7) in slot c ^ 2(r & 7).  V
+    static_assert(HD == 128 || HD == 64, "k_slot; a wave's V dims in one lane group");
+    // K planes: row r's chunk c (dims 8c..8c+7) in slot c ^ 2(r & 7) (rows of
+    // 256 bytes) or c ^ (r & 6) (of 128).  V
     // planes: dim d's chunk g (the keys lane group g supplies) in slot g ^
     // v_swz(d).  A 64-lane ds_read_b128 is served in four cycles of 16 lanes of
     // a half-wave that agree in the parity of lane bits 2-4 (bit 0 may also
@@ -124,7 +125,7 @@ __global__ __launch_bounds__(64 * QS * HW * KSP, 2) void prefill_split_kernel(
         uint4 v[NB * KSP][3][PL];
         float raw[2 * KSP * PL * 8];  // f32 K and V of the next step's tiles
     } sm;
-    auto k_slot = [](int r, int c) { return r * KC + (c ^ ((r & 7) << 1)); };
+    auto k_slot = [](int r, int c) { return r * KC + (c ^ (HD == 128 ? (r & 7) << 1 : r & 6)); };
     auto v_swz = [](int d) { return ((d >> 4) & 1) | (((d >> 2) & 1) << 1); };
 
     const int tid = threadIdx.x;
@@ -551,23 +552,33 @@ __global__ __launch_bounds__(64 * QS * HW * KSP, 2) void prefill_split_kernel(
     }
 }
 
-template <int HW, int QS, int KSP, bool PAIR>
+template <int HD, int HW, int QS, int KSP, bool PAIR>
 hipError_t launch_t(const Shape& s, const SplitParams& pp, hipStream_t st) {
     const int groups = ((pp.n + 15) / 16 + QS - 1) / QS;
-    hipLaunchKernelGGL((prefill_split_kernel<128, HW, QS, KSP, PAIR>),
+    hipLaunchKernelGGL((prefill_split_kernel<HD, HW, QS, KSP, PAIR>),
                        dim3(groups * (s.num_heads / HW)), dim3(64 * QS * HW * KSP), 0, st, pp);
     return hipGetLastError();
 }
 
-template <int HW>
+template <int HD, int HW>
 hipError_t launch_hw(const Shape& s, const SplitParams& pp, PrefillSplit form, hipStream_t st) {
     switch (form) {
-        case PrefillSplit::kKeySplit: return launch_t<HW, 4 / HW, 2, true>(s, pp, st);
-        case PrefillSplit::kPaired: return launch_t<HW, 8 / HW, 1, true>(s, pp, st);
-        case PrefillSplit::kConsecutive: return launch_t<HW, 8 / HW, 1, false>(s, pp, st);
+        case PrefillSplit::kKeySplit: return launch_t<HD, HW, 4 / HW, 2, true>(s, pp, st);
+        case PrefillSplit::kPaired: return launch_t<HD, HW, 8 / HW, 1, true>(s, pp, st);
+        case PrefillSplit::kConsecutive: return launch_t<HD, HW, 8 / HW, 1, false>(s, pp, st);
         case PrefillSplit::kNone: break;
     }
     return hipErrorInvalidValue;
+}
+
+template <int HD>
+hipError_t launch_hd(const Shape& s, const SplitParams& pp, PrefillSplit form, hipStream_t st) {
+    // four heads on the tiles where there are so many: 4096 rows of the
+    // Llama-3-8B shape 672 against 690 us with two
+    if (form == PrefillSplit::kConsecutive && s.kv_mul % 4 == 0)
+        return launch_t<HD, 4, 2, 1, false>(s, pp, st);
+    return s.kv_mul % 2 == 0 ? launch_hw<HD, 2>(s, pp, form, st)
+                             : launch_hw<HD, 1>(s, pp, form, st);
 }
 
 }  // namespace
@@ -577,12 +588,11 @@ hipError_t launch_prefill_split(const Shape& s, const PrefillArgs& a, PrefillSpl
     SplitParams pp{a.q,   a.k_cache, a.v_cache,   a.cos_t,  a.sin_t,  a.out, a.start,
                    a.n,   s.dim,     s.num_heads, s.kv_dim, s.kv_mul, s.half,
                    1.4426950408889634f / sqrtf((float)s.head_dim)};
-    if (s.head_dim != 128) return hipErrorInvalidValue;
-    // four heads on the tiles where there are so many: 4096 rows of the
-    // Llama-3-8B shape 672 against 690 us with two
-    if (form == PrefillSplit::kConsecutive && s.kv_mul % 4 == 0)
-        return launch_t<4, 2, 1, false>(s, pp, st);
-    return s.kv_mul % 2 == 0 ? launch_hw<2>(s, pp, form, st) : launch_hw<1>(s, pp, form, st);
+    switch (s.head_dim) {
+        case 64: return launch_hd<64>(s, pp, form, st);
+        case 128: return launch_hd<128>(s, pp, form, st);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 }  // namespace slm

@@ -1,4 +1,4 @@
-"""The split-bf16 prefill (head_dim 128) at the sizes where its forms, blocks
+"""The split-bf16 prefill (head_dim 64 and 128) at the sizes where its forms, blocks
 and key tiles begin and end, against float64 attention, and with values that
 cannot be split."""
 import numpy as np
@@ -9,13 +9,12 @@ from slm_testlib import gen, load_product
 P = load_product()
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
-HD = 128
 
 
 def run(heads, kvh, start, q, k, v):
-    """attend_batch of rotated q [n][heads*HD] over cache rows 0..start+n-1."""
+    """attend_batch of rotated q [n][dim] over cache rows 0..start+n-1."""
     rows, n = k.shape[0], q.shape[0]
-    with P.AttentionContext(heads * HD, heads, kvh, max(rows, 16), 1) as ctx:
+    with P.AttentionContext(q.shape[1], heads, kvh, max(rows, 16), 1) as ctx:
         ctx.kv_write(0, 0, 0, k)
         ctx.kv_write(0, 1, 0, v)
         qd = torch.from_numpy(q).cuda()
@@ -28,13 +27,13 @@ def run(heads, kvh, start, q, k, v):
 
 def attend64(heads, kvh, start, q, k, v):
     """float64 attention; (out, per-element sum of |p v|, largest |score|)."""
-    n = q.shape[0]
+    n, hd = q.shape[0], q.shape[1] // heads
     out, mag, smax = np.empty(q.shape), np.empty(q.shape), 0.0
     mask = np.arange(k.shape[0])[None, :] > start + np.arange(n)[:, None]
     for h in range(heads):
         g = h // (heads // kvh)
-        hs, gs = slice(h * HD, (h + 1) * HD), slice(g * HD, (g + 1) * HD)
-        s = q[:, hs].astype(np.float64) @ k[:, gs].astype(np.float64).T / np.sqrt(HD)
+        hs, gs = slice(h * hd, (h + 1) * hd), slice(g * hd, (g + 1) * hd)
+        s = q[:, hs].astype(np.float64) @ k[:, gs].astype(np.float64).T / np.sqrt(hd)
         s[mask] = -np.inf
         smax = max(smax, np.abs(s[~mask]).max())
         p = np.exp(s - s.max(1, keepdims=True))
@@ -44,23 +43,26 @@ def attend64(heads, kvh, start, q, k, v):
     return out, mag, smax
 
 
-# heads, kv_heads, start, n: one, two, three, four and eight heads per KV head;
+# hd, heads, kv_heads, start, n: one, two, three, four and eight heads per KV head;
 # key splits, paired and consecutive blocks; block and tile edges (15/16/17
 # rows, 127 to 129 and 159 to 161 keys), odd and even block counts
 CASES = [
-    (2, 1, 112, 16), (2, 1, 111, 17), (2, 1, 113, 15), (4, 1, 0, 128), (4, 1, 0, 129),
-    (1, 1, 100, 28), (1, 1, 127, 33), (3, 1, 0, 160), (3, 3, 30, 131), (8, 1, 96, 65),
-    (12, 4, 0, 250), (2, 2, 1000, 2), (4, 2, 500, 47),
-    (32, 8, 0, 545), (32, 32, 3, 528), (32, 8, 0, 1025), (24, 8, 40, 1400), (32, 16, 0, 1040),
+    (128, 2, 1, 112, 16), (128, 2, 1, 111, 17), (128, 2, 1, 113, 15), (128, 4, 1, 0, 128),
+    (128, 4, 1, 0, 129), (128, 1, 1, 100, 28), (128, 1, 1, 127, 33), (128, 3, 1, 0, 160),
+    (128, 3, 3, 30, 131), (128, 8, 1, 96, 65), (128, 12, 4, 0, 250), (128, 2, 2, 1000, 2),
+    (128, 4, 2, 500, 47), (128, 32, 8, 0, 545), (128, 32, 32, 3, 528), (128, 32, 8, 0, 1025),
+    (128, 24, 8, 40, 1400), (128, 32, 16, 0, 1040),
+    (64, 32, 8, 0, 380), (64, 32, 8, 0, 384), (64, 24, 8, 5, 511), (64, 32, 8, 1, 1023),
+    (64, 32, 32, 0, 1040), (64, 36, 12, 0, 1100), (64, 32, 8, 0, 2065), (64, 48, 6, 3, 1403),
 ]
 
 
-@pytest.mark.parametrize("heads,kvh,start,n", CASES)
-def test_against_float64(heads, kvh, start, n):
+@pytest.mark.parametrize("hd,heads,kvh,start,n", CASES)
+def test_against_float64(hd, heads, kvh, start, n):
     rows = start + n
-    q = gen([71, heads, start, n], (n, heads * HD)) * np.float32(4)
-    k = gen([72, heads, start, n], (rows, kvh * HD)) * np.float32(2)
-    v = gen([73, heads, start, n], (rows, kvh * HD))
+    q = gen([71, heads, start, n], (n, heads * hd)) * np.float32(4)
+    k = gen([72, heads, start, n], (rows, kvh * hd)) * np.float32(2)
+    v = gen([73, heads, start, n], (rows, kvh * hd))
     ref, mag, smax = attend64(heads, kvh, start, q, k, v)
     got = run(heads, kvh, start, q, k, v)
     # Roundings of 2^-24: six per 32-key tile in an output sum and one in the
@@ -76,31 +78,32 @@ def test_against_float64(heads, kvh, start, n):
     assert rel < 3e-6, rel
 
 
-@pytest.mark.parametrize("heads,kvh,start,n", [(2, 1, 100, 60), (32, 8, 0, 600), (32, 32, 0, 1100)])
-def test_values_that_cannot_be_split(heads, kvh, start, n):
+@pytest.mark.parametrize("hd,heads,kvh,start,n", [(128, 2, 1, 100, 60), (128, 32, 8, 0, 600),
+                                                  (128, 32, 32, 0, 1100), (64, 32, 8, 0, 500)])
+def test_values_that_cannot_be_split(hd, heads, kvh, start, n):
     """-inf scores drop their key, inf and near-overflow values travel, and
     earlier rows and other KV heads do not see them."""
     rows = start + n
-    q = np.abs(gen([74, n], (n, heads * HD))) + np.float32(0.1)
-    k = gen([75, n], (rows, kvh * HD))
-    v = gen([76, n], (rows, kvh * HD))
+    q = np.abs(gen([74, n], (n, heads * hd))) + np.float32(0.1)
+    k = gen([75, n], (rows, kvh * hd))
+    v = gen([76, n], (rows, kvh * hd))
     j_k, j_v, j_big = rows - 45, rows - 20, rows - 9
     # its probability stays small beside a running max that may lag by 2^8
-    k[j_big, :HD] = -2
+    k[j_big, :hd] = -2
     k2, v2 = k.copy(), v.copy()
-    k2[j_k, :HD] = -np.inf           # every score of KV head 0 there is -inf
+    k2[j_k, :hd] = -np.inf           # every score of KV head 0 there is -inf
     v2[j_v, 3] = np.inf
     v2[j_big, 5] = np.float32(3.4e38)  # rounds to a bf16 infinity
     got = run(heads, kvh, start, q, k2, v2)
     kr = k.copy()
-    kr[j_k, :HD] = np.float32(-1e4)  # exp underflows to 0: the key drops out
+    kr[j_k, :hd] = np.float32(-1e4)  # exp underflows to 0: the key drops out
     vr = v.copy()
     vr[j_v, 3] = 0
     vr[j_big, 5] = 0
     ref, mag, _ = attend64(heads, kvh, start, q, kr, vr)
     pos = start + np.arange(n)
     per = heads // kvh
-    cols0 = np.arange(per) * HD      # KV head 0's query heads
+    cols0 = np.arange(per) * hd      # KV head 0's query heads
     assert np.isposinf(got[np.ix_(pos >= j_v, cols0 + 3)]).all()
     big = got[np.ix_(pos >= j_big, cols0 + 5)]
     assert np.isfinite(big).all() and (big > 1e30).all()
