@@ -48,8 +48,8 @@ __device__ __forceinline__ floatx4 mfma4(float a, float b, floatx4 c) {
 
 struct PrefillParams {
     const float* q;
-    const float* k_cache;
-    const float* v_cache;
+    float* k_cache;
+    float* v_cache;
     const float* cos_t;
     const float* sin_t;
     float* out;
@@ -61,6 +61,8 @@ struct PrefillParams {
     int kv_mul;
     int half;
     float scale_log2;
+    const float* k_new;  // [n][kv_dim] to append first, or nullptr
+    const float* v_new;
 };
 
 // LDS tile layouts.  Measured on MI355X with the bank-conflict counter over
@@ -208,6 +210,24 @@ prefill_mfma_kernel(PrefillParams p) {
     const int n_tiles = (kv_len + kKT - 1) / kKT;
     const int wave_rows = max(0, min(QPW, p.n - q0));
     const int wave_last_pos = p.start + q0 + wave_rows - 1;
+
+    // The batch's rows of this KV head into the cache (prefill_appends(): the
+    // only workgroup that writes or reads them), as kv_append_kernel does.
+    if (p.k_new != nullptr) {
+        for (int i = tid; i < p.n * (HD / 2); i += NT) {
+            const int r = i / (HD / 2), j = i % (HD / 2);
+            const long at = (long)r * p.kv_dim + g * HD + 2 * j;
+            const long to = (long)p.start * p.kv_dim + at;
+            const float2 kk = *reinterpret_cast<const float2*>(p.k_new + at);
+            const long tr = (long)(p.start + r) * p.half + j;
+            *reinterpret_cast<float2*>(p.k_cache + to) =
+                rope_pair_exact(kk, p.cos_t[tr], p.sin_t[tr]);
+            *reinterpret_cast<float2*>(p.v_cache + to) =
+                *reinterpret_cast<const float2*>(p.v_new + at);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    }
 
     // Q fragments: row q0 + qt*16 + lr, dims lg*DPL .. +DPL, rotated, scaled.
     // All q and table loads are issued before the first use (a load inside
@@ -659,7 +679,11 @@ bool head_dim_supported(int hd) {
 hipError_t launch_prefill_mfma(const Shape& s, const PrefillArgs& a, hipStream_t st) {
     PrefillParams pp{a.q,   a.k_cache, a.v_cache,   a.cos_t,  a.sin_t,  a.out, a.start,
                      a.n,   s.dim,     s.num_heads, s.kv_dim, s.kv_mul, s.half,
-                     1.4426950408889634f / sqrtf((float)s.head_dim)};
+                     1.4426950408889634f / sqrtf((float)s.head_dim), a.k_new, a.v_new};
+    if (a.k_new != nullptr &&
+        (a.v_new == nullptr || a.cos_t == nullptr || a.sin_t == nullptr ||
+         !prefill_appends(s.head_dim, s.num_heads, s.kv_mul, s.cus, a.start, a.n)))
+        return hipErrorInvalidValue;
     if (a.n > 65535 * 64) return hipErrorInvalidValue;
     const PrefillSplit split =
         prefill_split_plan(s.head_dim, s.num_heads, s.kv_mul, s.cus, a.start, a.n);

@@ -315,6 +315,22 @@ int do_attend(slm_attn_ctx* c, int layer, int start, int n, const float* q,
     return launch_status(c, e, "prefill kernel launch");
 }
 
+// K/V append and attention of a prefill batch, q and k un-rotated.
+int do_prefill(slm_attn_ctx* c, int layer, int start, int n, const float* q, const float* k,
+               const float* v, float* out) {
+    const slm::Shape& s = c->shape;
+    if (!slm::prefill_appends(s.head_dim, s.num_heads, s.kv_mul, s.cus, start, n)) {
+        const int rc = do_append(c, layer, start, n, k, v);
+        return rc ? rc : do_attend(c, layer, start, n, q, out, true);
+    }
+    slm::PrefillArgs pa{q,   k_base(c, layer), v_base(c, layer), c->cos_t, c->sin_t, out, start, n,
+                        k,   v};
+    Timed t(c, SLM_K_PREFILL);
+    hipError_t e = slm::launch_prefill_mfma(s, pa, c->stream);
+    t.done();
+    return launch_status(c, e, "prefill kernel launch");
+}
+
 int ensure_stage(slm_attn_ctx* c, size_t floats) {
     if (c->stage_floats >= floats) return SLM_OK;
     if (c->capturing) return refuse_capture(c, "host staging buffer");
@@ -781,8 +797,7 @@ int slm_attn_prefill_dev(slm_attn_ctx* c, int32_t layer, int32_t start,
     if ((rc = check_out_alias(c, out, qn, {{q, qn}, {k, kn}, {v, kn}}, true)) ||
         (rc = check_in_not_kv(c, {{q, qn}, {k, kn}, {v, kn}})))
         return rc;
-    if ((rc = do_append(c, layer, start, n, k, v))) return rc;
-    return do_attend(c, layer, start, n, q, out, true);
+    return do_prefill(c, layer, start, n, q, k, v, out);
 }
 
 int slm_attn_decode(slm_attn_ctx* c, int32_t layer, int32_t pos, const float* q,
@@ -1136,8 +1151,7 @@ int slm_attn_prefill_xb_dev(slm_attn_ctx* c, int32_t layer, int32_t start, int32
     if ((rc = project_qkv(c, n, xb, wq, wk, wv, &q, &k, &v))) return rc;
     if (overlaps(out, rows * 4, c->qkv, c->qkv_floats * 4))
         return fail(c, SLM_ERR_ALIAS, "out must not overlap the context's buffers");
-    if ((rc = do_append(c, layer, start, n, k, v))) return rc;
-    return do_attend(c, layer, start, n, q, out, true);
+    return do_prefill(c, layer, start, n, q, k, v, out);
 }
 
 int slm_attn_decode_wo_dev(slm_attn_ctx* c, int32_t layer, int32_t pos, float* xb,
@@ -1167,8 +1181,7 @@ int slm_attn_prefill_wo_dev(slm_attn_ctx* c, int32_t layer, int32_t start, int32
         return rc;
     float *q, *k, *v;
     if ((rc = project_qkv(c, n, xb, wq, wk, wv, &q, &k, &v))) return rc;
-    if ((rc = do_append(c, layer, start, n, k, v))) return rc;
-    if ((rc = do_attend(c, layer, start, n, q, xb, true))) return rc;
+    if ((rc = do_prefill(c, layer, start, n, q, k, v, xb))) return rc;
     return project(c, wo, xb, n, x_mid, x);
 }
 

@@ -208,6 +208,8 @@ int do_decode(slm_attn_ctx* c, int layer, int pos, const float* q, const float* 
 int do_decode_in(slm_attn_ctx* c, int layer, int pos, const float* q, const float* k_new,
                  const float* v_new, float* out, bool rotate, float* part_o, float* part_ml,
                  bool timed);
+int do_prefill(slm_attn_ctx* c, int layer, int start, int n, const float* q, const float* k,
+               const float* v, float* out);
 int do_attend(slm_attn_ctx* c, int layer, int start, int n, const float* q, float* out,
               bool rotate);
 int ensure_q8(slm_attn_ctx* c, size_t n, int nb);

@@ -73,13 +73,17 @@ hipError_t launch_decode_combine(const Shape& s, const DecodeArgs& a, hipStream_
 // attend to cache rows 0..start+b.  q is un-rotated when cos_t != nullptr.
 struct PrefillArgs {
     const float* q;
-    const float* k_cache;
-    const float* v_cache;
+    float* k_cache;
+    float* v_cache;
     const float* cos_t;
     const float* sin_t;
     float* out;
     int start;
     int n;
+    // (launch_prefill_mfma, where prefill_appends()) the batch's K and V rows
+    // [n][kv_dim], which the kernel then appends at start first
+    const float* k_new = nullptr;
+    const float* v_new = nullptr;
 };
 hipError_t launch_prefill_mfma(const Shape& s, const PrefillArgs& a,
                                hipStream_t st);

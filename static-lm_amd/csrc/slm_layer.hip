@@ -173,9 +173,7 @@ int slm_layer_forward_dev(slm_attn_ctx* c, int32_t layer, int32_t start, int32_t
     if (one) {
         if ((rc = do_decode(c, layer, start, q, k, v, att, true))) return rc;
     } else {
-        if ((rc = do_append(c, layer, start, n, k, v)) ||
-            (rc = do_attend(c, layer, start, n, q, att, true)))
-            return rc;
+        if ((rc = do_prefill(c, layer, start, n, q, k, v, att))) return rc;
     }
     // x_mid = x + Wo . att (:445-446 / 595-605)
     if ((rc = project(c, w->wo, att, n, x_mid, x))) return rc;
