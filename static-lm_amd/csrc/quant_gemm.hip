@@ -39,6 +39,7 @@ namespace slm {
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 
 // A token's GEMV reads each weight once: nontemporal loads stream them past
@@ -689,15 +690,16 @@ __global__ __launch_bounds__(256) void gemv_q8in_swiglu_kernel(GemvSwigluParams 
 
 // ---- MFMA GEMM: batches of 5 or more tokens ----
 //
-// Workgroup tile 64 rows x 64 tokens, four waves of 32 x 32 (2 x 2 tiles of
-// v_mfma_i32_16x16x32_i8, one Q-block of K = 32 per instruction).  Lane l
-// feeds A[l%16][8*(l/16)..+7] = weights 8g..8g+7 of row l%16 (g = l/16) and
-// B[8g..+7][l%16] = the same eight activations of token l%16, and holds
-// D[4g+j][l%16].  Per block each element gets acc = acc + float(D) * (dw*da).
-// The kernel is bound by that f32 epilogue (VALU), so everything else that
-// costs VALU is done once per workgroup at staging: the nibbles are widened
-// to i8 weights (in weight order, so a fragment is one 8-byte read) and the
-// weight scales to f32.
+// Workgroup tile 64 rows x 64 tokens, four waves of 32 x 32, or 128 x 128,
+// eight waves of 32 x 64, in tiles of v_mfma_i32_32x32x32_i8, one Q-block of K
+// = 32 per instruction (twice the rate of the 16x16x32 form).  Lane l (l32 =
+// l%32, h = l/32) feeds weights 16h..16h+15 of row l32 and the same sixteen
+// activations of token l32, and holds row 8a + 4h + b of token l32 in register
+// 4a + b.  Per block each element gets acc = acc + float(D) * (dw*da).  The
+// kernel is bound by that f32 epilogue (VALU), so everything else that costs
+// VALU is done once per workgroup at staging: the nibbles are widened to i8
+// weights (in weight order, so a fragment is one 16-byte read) and the weight
+// scales to f32.
 
 struct GemmParams {
     QMat m[3];
@@ -718,10 +720,12 @@ __device__ __forceinline__ uint32_t nib_to_i8(uint32_t x) {
 }
 
 // LDS stage of the GEMM: kScaleChunk blocks of the workgroup's RT weight rows
-// (widened to i8) and TT tokens.  Row strides are padded to 68 dwords so that
-// the 8-byte fragment reads of a half-wave (16 rows or tokens x 2 lane
-// groups) hit 64 different banks; scales are stored block-major so a lane's
-// four rows are one 16-byte read.
+// (widened to i8) and TT tokens.  Row strides are padded to 68 dwords (17
+// chunks of 16 bytes) so that the 16-byte fragment reads of rows r and r + 16
+// alone share banks, and those are never served in one cycle (a 64-lane
+// ds_read_b128 takes four, each 16 lanes of a half-wave with the same parity
+// of lane bits 2-4); scales are stored block-major so a lane's four
+// consecutive rows are one 16-byte read.
 constexpr int kAStride = 68;  // dwords per weight row: 8 blocks x 32 i8 + pad
 constexpr int kBStride = 68;  // dwords per token: 8 blocks x 32 B + pad
 template <int RT, int TT>
@@ -732,20 +736,33 @@ struct GemmStage {
     float da[kScaleChunk][TT];
 };
 
-// Workgroup shapes: WRW x WTW waves, each 32 rows x 16*NTS tokens.  64 x 64
-// (2 x 2 waves of 32 x 32), or 128 x 128 (4 x 2 waves of 32 x 64) for
-// products with enough tiles to fill the CUs (launch_q4_gemm), where each
-// lane's 32 outputs share the block's
-// fragment and scale reads twice as widely (the loop's VALU cost per output
-// element and block falls from ~5.6 to ~4.9 ops, against the epilogue's 4).
+// Workgroup shapes: WRW x WTW waves, each 32 rows x 32*NTS tokens.  64 x 64 (2
+// x 2 waves of 32 x 32), or 128 x 128 (4 x 2 waves of 32 x 64) for products with
+// enough tiles to fill the CUs (launch_q4_gemm), where each lane's 32 outputs
+// share the block's weight fragment and scale reads.
 template <int WRW, int WTW, int NTS>
 struct GemmShape {
     static constexpr int NW = WRW * WTW;
     static constexpr int NT = 64 * NW;
     static constexpr int RT = 32 * WRW;       // rows per workgroup
-    static constexpr int TT = 16 * NTS * WTW;  // tokens per workgroup
+    static constexpr int TT = 32 * NTS * WTW;  // tokens per workgroup
     static_assert(RT == NT / 4 && TT == NT / 4, "one row and one token per thread quad");
 };
+
+// A block's integer sum (|isum| <= 32 * 8 * 127) as f32: with the accumulator
+// started at the bits of 1.5 * 2^23 the result's bits are those of 1.5 * 2^23
+// + isum, and one exact subtraction leaves isum.  v_cvt_f32_i32 issues at half
+// the rate of v_sub_f32 (4.3 against 2.4 cycles per wave, two waves per SIMD).
+// Used where the kernel is bound by that (128 x 128 tiles; 2048 tokens, convert
+// against subtract: gate/up 1005 against 986 us, Wo 147 against 140); the 64 x
+// 64 tiles, bound by latency, are better without the sixteen base registers
+// (512 tokens: gate/up 278 against 283).
+constexpr int kSumBits = 0x4B400000;
+constexpr float kSumBase = 12582912.0f;
+template <bool SUB>
+__device__ __forceinline__ float sum_f32(int d) {
+    return SUB ? __int_as_float(d) - kSumBase : (float)d;
+}
 
 template <int WRW, int WTW, int NTS>
 __global__ __launch_bounds__(64 * WRW * WTW) void gemm_q4_mfma_kernel(GemmParams p) {
@@ -756,8 +773,8 @@ __global__ __launch_bounds__(64 * WRW * WTW) void gemm_q4_mfma_kernel(GemmParams
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
-    const int lr = lane & 15;
-    const int g = lane >> 4;
+    const int l32 = lane & 31;
+    const int hh = lane >> 5;
 
     // workgroup -> (matrix, row tile, token tile); token tiles vary fastest
     const int n_tt = (p.batch + TT - 1) / TT;
@@ -842,16 +859,20 @@ __global__ __launch_bounds__(64 * WRW * WTW) void gemm_q4_mfma_kernel(GemmParams
         }                                                                                 \
     } while (0)
 
-    // this wave's 32 rows x 16*NTS tokens
-    const int qr = (wave % WRW) * 32, qt = (wave / WRW) * (16 * NTS);
+    // this wave's 32 rows x 32*NTS tokens
+    const int qr = (wave % WRW) * 32, qt = (wave / WRW) * (32 * NTS);
 
-    float acc[2][NTS][4];
+    constexpr bool SUB = NTS > 1;
+    float acc[NTS][16];
+    v16i base;
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int j = 0; j < 16; ++j) {
+        base[j] = SUB ? kSumBits : 0;
 #pragma unroll
-        for (int b = 0; b < NTS; ++b)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[a][b][j] = 0.0f;
+        for (int b = 0; b < NTS; ++b) acc[b][j] = 0.0f;
+    }
+
+    if constexpr (SUB) asm("" : "+v"(base));  // kept, not rebuilt for every block
 
     SLM_GEMM_LOAD_STAGE(0);
     SLM_GEMM_STORE_STAGE(st[0]);
@@ -864,49 +885,36 @@ __global__ __launch_bounds__(64 * WRW * WTW) void gemm_q4_mfma_kernel(GemmParams
 #pragma unroll
         for (int kb = 0; kb < kScaleChunk; ++kb) {
             if (b0 + kb >= nb) break;  // uniform
-            long af[2], bf[NTS];
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                const uint2 w = *reinterpret_cast<const uint2*>(
-                    &S.a[(qr + 16 * s + lr) * kAStride + kb * 8 + 2 * g]);
-                af[s] = (long)(((uint64_t)w.y << 32) | w.x);
-            }
+            const v4i af = *reinterpret_cast<const v4i*>(
+                &S.a[(qr + l32) * kAStride + kb * 8 + 4 * hh]);
+            v16i d[NTS];
+            float da[NTS];
 #pragma unroll
             for (int s = 0; s < NTS; ++s) {
-                const uint2 x = *reinterpret_cast<const uint2*>(
-                    &S.b[(qt + 16 * s + lr) * kBStride + kb * 8 + 2 * g]);
-                bf[s] = (long)(((uint64_t)x.y << 32) | x.x);
+                const v4i bf = *reinterpret_cast<const v4i*>(
+                    &S.b[(qt + 32 * s + l32) * kBStride + kb * 8 + 4 * hh]);
+                d[s] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, bf, base, 0, 0, 0);
+                da[s] = S.da[kb][qt + 32 * s + l32];
             }
-            v4i d[2][NTS];
-#pragma unroll
-            for (int rs2 = 0; rs2 < 2; ++rs2)
-#pragma unroll
-                for (int ts = 0; ts < NTS; ++ts)
-                    d[rs2][ts] = __builtin_amdgcn_mfma_i32_16x16x32_i8(af[rs2], bf[ts],
-                                                                       v4i{0, 0, 0, 0}, 0, 0, 0);
             // the scale products stay on the VALU: on the matrix cores (an
             // f16 or f32 MFMA whose K = 0 slice holds the two scales, exact)
             // the epilogue waits for them and the kernel ran slower
-            float dw[2][4], da[NTS];
+            float dw[16];
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                const float4 h = *reinterpret_cast<const float4*>(&S.dw[kb][qr + 16 * s + 4 * g]);
-                dw[s][0] = h.x;
-                dw[s][1] = h.y;
-                dw[s][2] = h.z;
-                dw[s][3] = h.w;
+            for (int a = 0; a < 4; ++a) {
+                const float4 h = *reinterpret_cast<const float4*>(&S.dw[kb][qr + 8 * a + 4 * hh]);
+                dw[4 * a + 0] = h.x;
+                dw[4 * a + 1] = h.y;
+                dw[4 * a + 2] = h.z;
+                dw[4 * a + 3] = h.w;
             }
 #pragma unroll
-            for (int s = 0; s < NTS; ++s) da[s] = S.da[kb][qt + 16 * s + lr];
+            for (int s = 0; s < NTS; ++s)
 #pragma unroll
-            for (int rs2 = 0; rs2 < 2; ++rs2)
-#pragma unroll
-                for (int ts = 0; ts < NTS; ++ts)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const float sc = dw[rs2][j] * da[ts];
-                        acc[rs2][ts][j] = acc[rs2][ts][j] + (float)d[rs2][ts][j] * sc;
-                    }
+                for (int j = 0; j < 16; ++j) {
+                    const float sc = dw[j] * da[s];
+                    acc[s][j] = acc[s][j] + sum_f32<SUB>(d[s][j]) * sc;
+                }
         }
         if (sg + 1 < n_stages) SLM_GEMM_STORE_STAGE(st[(sg + 1) & 1]);
     }
@@ -919,51 +927,50 @@ __global__ __launch_bounds__(64 * WRW * WTW) void gemm_q4_mfma_kernel(GemmParams
     const bool vec = (M.rows & 3) == 0 && (M.out_stride & 3) == 0 &&
                      ((reinterpret_cast<uintptr_t>(M.out) | reinterpret_cast<uintptr_t>(M.res)) &
                       15) == 0;
+    const int rb = wr0 + qr + 4 * hh;  // this lane's rows: rb + 8a + (0..3)
     if (vec) {
-        float4 rv[2][NTS];
+        float4 rv[NTS][4];
         if (M.res) {
 #pragma unroll
-            for (int rs2 = 0; rs2 < 2; ++rs2)
+            for (int s = 0; s < NTS; ++s)
 #pragma unroll
-                for (int ts = 0; ts < NTS; ++ts) {
-                    const int t = min(wt0 + qt + 16 * ts + lr, p.batch - 1);
-                    const int r0 = min(wr0 + qr + 16 * rs2 + 4 * g, M.rows - 4);
-                    rv[rs2][ts] = ld4(M.res + (long)t * M.out_stride + r0);
+                for (int a = 0; a < 4; ++a) {
+                    const int t = min(wt0 + qt + 32 * s + l32, p.batch - 1);
+                    const int r0 = min(rb + 8 * a, M.rows - 4);
+                    rv[s][a] = ld4(M.res + (long)t * M.out_stride + r0);
                 }
         }
 #pragma unroll
-        for (int rs2 = 0; rs2 < 2; ++rs2)
+        for (int s = 0; s < NTS; ++s)
 #pragma unroll
-            for (int ts = 0; ts < NTS; ++ts) {
-                const int t = wt0 + qt + 16 * ts + lr;
-                const int r0 = wr0 + qr + 16 * rs2 + 4 * g;
+            for (int a = 0; a < 4; ++a) {
+                const int t = wt0 + qt + 32 * s + l32;
+                const int r0 = rb + 8 * a;
                 if (t >= p.batch || r0 >= M.rows) continue;
-                float4 y = make_float4(acc[rs2][ts][0], acc[rs2][ts][1], acc[rs2][ts][2],
-                                       acc[rs2][ts][3]);
+                float4 y = make_float4(acc[s][4 * a], acc[s][4 * a + 1], acc[s][4 * a + 2],
+                                       acc[s][4 * a + 3]);
                 if (M.res) {
-                    y.x = rv[rs2][ts].x + y.x;
-                    y.y = rv[rs2][ts].y + y.y;
-                    y.z = rv[rs2][ts].z + y.z;
-                    y.w = rv[rs2][ts].w + y.w;
+                    y.x = rv[s][a].x + y.x;
+                    y.y = rv[s][a].y + y.y;
+                    y.z = rv[s][a].z + y.z;
+                    y.w = rv[s][a].w + y.w;
                 }
                 *reinterpret_cast<float4*>(M.out + (long)t * M.out_stride + r0) = y;
             }
         return;
     }
 #pragma unroll
-    for (int rs2 = 0; rs2 < 2; ++rs2)
+    for (int s = 0; s < NTS; ++s) {
+        const int t = wt0 + qt + 32 * s + l32;
+        if (t >= p.batch) continue;
 #pragma unroll
-        for (int ts = 0; ts < NTS; ++ts) {
-            const int t = wt0 + qt + 16 * ts + lr;
-            if (t >= p.batch) continue;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int r = wr0 + qr + 16 * rs2 + 4 * g + j;
-                if (r >= M.rows) continue;
-                const long o = (long)t * M.out_stride + r;
-                M.out[o] = M.res ? M.res[o] + acc[rs2][ts][j] : acc[rs2][ts][j];
-            }
+        for (int j = 0; j < 16; ++j) {
+            const int r = rb + 8 * (j >> 2) + (j & 3);
+            if (r >= M.rows) continue;
+            const long o = (long)t * M.out_stride + r;
+            M.out[o] = M.res ? M.res[o] + acc[s][j] : acc[s][j];
         }
+    }
 }
 #undef SLM_GEMM_LOAD_STAGE
 #undef SLM_GEMM_STORE_STAGE
@@ -1397,9 +1404,10 @@ long device_cus() {
 // 36.2 against 27 / 43; 576 x 1536, 130 / 512 tokens (324 / 1152) 17.2 / 17.8 against
 // 10.1 / 18.7.
 //
-// Otherwise 128 x 128 workgroups (one per CU; 10% less VALU per output
-// element and block, measured on the 4096-token Q/K/V GEMM: 0.48 against
-// 0.53 ms) or 64 x 64 (two per CU).  The estimate of each is the workgroups
+// Otherwise 128 x 128 workgroups (one per CU; less VALU per output element and
+// block) or 64 x 64 (two per CU).  On 32x32x32 MFMAs (against 16x16x32 ones, which
+// took twice the matrix cycles) 2048 tokens take, before and after: gate/up 1035
+// -> 986 us, Q/K/V 223 -> 206, down 497 -> 454, Wo 153 -> 140.  The estimate of each is the workgroups
 // a CU runs in turn times one workgroup's work; products with few big tiles
 // would leave CUs idle (Wo at 512 tokens: 128 workgroups of 128 x 128 on 256
 // CUs).  Tile shape does not change results (each output is one thread's
@@ -1418,8 +1426,8 @@ hipError_t launch_q4_gemm(const Q4Job* jobs, int njobs, const uint32_t* aq, cons
     const double t128 = (double)((w128 + cus - 1) / cus) * 4.0;
     const double t64 = (double)((w64 + cus - 1) / cus) * 1.1;
     if (w16 <= 4 * cus) return launch_gemm_small(jobs, njobs, aq, ad, nb, batch, st);
-    return t128 < t64 ? launch_gemm_t<4, 2, 4>(jobs, njobs, aq, ad, nb, batch, st)
-                      : launch_gemm_t<2, 2, 2>(jobs, njobs, aq, ad, nb, batch, st);
+    return t128 < t64 ? launch_gemm_t<4, 2, 2>(jobs, njobs, aq, ad, nb, batch, st)
+                      : launch_gemm_t<2, 2, 1>(jobs, njobs, aq, ad, nb, batch, st);
 }
 
 }  // namespace slm
