@@ -50,10 +50,14 @@ struct NormArgs {
 
 // Rows of n % 32 == 0: quad q of the workgroup owns blocks q, q + 64, ...
 // (lane part p: elements 8p..8p+7 of each) in both phases, so x and w are
-// loaded once, up front, and held in registers across the chain.
+// loaded once, up front, and held in registers across the chain.  KP is the
+// row's passes rounded up to a power of two: the chains of one row keep one
+// lane group of one wave busy, so a batch of rows lives on how many
+// workgroups share a CU, and registers for eight passes (16384 elements)
+// left room for two (2048 rows of 4096: 29.2 us, now 19.4).
 constexpr int kNormMaxPasses = 8;  // n <= 64 blocks * 8 passes * 32 = 16384
 
-template <bool RMS>
+template <bool RMS, int KP>
 __global__ __launch_bounds__(kNormThreads) void norm_rows_kernel(NormArgs a) {
 #pragma clang fp contract(off)
     extern __shared__ __align__(16) float s_sq[];  // [4][norm_sq_stride(n)]
@@ -69,21 +73,25 @@ __global__ __launch_bounds__(kNormThreads) void norm_rows_kernel(NormArgs a) {
     const int nb = n / 32;
     const int passes = (nb + 63) / 64;
 
-    NormRow<kNormMaxPasses> r;
-    norm_row_load<kNormMaxPasses, RMS>(r, x, a.w, nb);
+    NormRow<KP> r;
+    norm_row_load<KP, RMS>(r, x, a.w, nb);
     norm_row_squares(r, nb, s_sq);
     __syncthreads();
-    norm_scale<RMS>(s_sq, st, vq, n, s_tail, a.eps, s_part, &s_scale);
+    // Wave w of a workgroup runs on SIMD w: the workgroups of a CU (256 apart
+    // on the whole device) give the chains to different waves.
+    const int rot = 64 * ((blockIdx.x + (blockIdx.x >> 8)) & 3);
+    norm_scale<RMS>(s_sq, st, vq, n, s_tail, a.eps, s_part, &s_scale,
+                    (tid + rot) & (kNormThreads - 1));
     __syncthreads();
     const float scale = s_scale;
 
 #pragma unroll
-    for (int k = 0; k < kNormMaxPasses; ++k) {
+    for (int k = 0; k < KP; ++k) {
         if (k >= passes) break;
         const int blk = (tid >> 2) + 64 * k;
         if (blk >= nb) break;  // uniform over the quad
         float4 f0, f1;
-        norm_row_values<kNormMaxPasses, RMS>(r, k, scale, &f0, &f1);
+        norm_row_values<KP, RMS>(r, k, scale, &f0, &f1);
         const int e0 = 32 * blk + 8 * part;
         if (a.out) {
             float* o = a.out + (long)blockIdx.x * a.out_stride + e0;
@@ -283,21 +291,35 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_parts_kernel(const Argm
     }
 }
 
+template <bool RMS, int KP>
+hipError_t launch_norm_rows(const NormArgs& a, int rows, size_t lds, hipStream_t st) {
+    if (lds > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(
+            reinterpret_cast<const void*>(norm_rows_kernel<RMS, KP>),
+            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((norm_rows_kernel<RMS, KP>), dim3(rows), dim3(kNormThreads), lds, st, a);
+    return hipGetLastError();
+}
+
 template <bool RMS>
 hipError_t launch_norm_t(const NormArgs& a, int rows, hipStream_t st) {
     const size_t lds = (size_t)4 * norm_sq_stride(a.n) * sizeof(float);
-    const bool blocks = a.n % 32 == 0;
-    const void* fn = blocks ? reinterpret_cast<const void*>(norm_rows_kernel<RMS>)
-                            : reinterpret_cast<const void*>(norm_rows_any_kernel<RMS>);
+    if (a.n % 32 == 0) {
+        const int passes = (a.n / 32 + 63) / 64;
+        if (passes <= 1) return launch_norm_rows<RMS, 1>(a, rows, lds, st);
+        if (passes <= 2) return launch_norm_rows<RMS, 2>(a, rows, lds, st);
+        if (passes <= 4) return launch_norm_rows<RMS, 4>(a, rows, lds, st);
+        return launch_norm_rows<RMS, kNormMaxPasses>(a, rows, lds, st);
+    }
     if (lds > 64 * 1024) {
-        const hipError_t e =
-            hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        const hipError_t e = hipFuncSetAttribute(
+            reinterpret_cast<const void*>(norm_rows_any_kernel<RMS>),
+            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    if (blocks)
-        hipLaunchKernelGGL(norm_rows_kernel<RMS>, dim3(rows), dim3(kNormThreads), lds, st, a);
-    else
-        hipLaunchKernelGGL(norm_rows_any_kernel<RMS>, dim3(rows), dim3(kNormThreads), lds, st, a);
+    hipLaunchKernelGGL(norm_rows_any_kernel<RMS>, dim3(rows), dim3(kNormThreads), lds, st, a);
     return hipGetLastError();
 }
 

@@ -90,18 +90,18 @@ __device__ __forceinline__ void norm_row_values(const NormRow<KP>& r, int k, flo
     *f1 = make_float4(v[4], v[5], v[6], v[7]);
 }
 
-// The four lane chains of the squares in s_sq (lanes 0..3 of wave 0), then
-// lane 0 combines them with the tail and returns the scale in s_scale.
+// The four lane chains of the squares in s_sq (threads tid 0..3, lanes of one
+// wave), then thread 0 combines them with the tail and returns the scale in
+// s_scale.
 // T terms are added while the next T are read from LDS (two buffers of T/4
 // float4 registers; a smaller T suits a kernel with other registers live).
 template <bool RMS, int T = 32>
 __device__ __forceinline__ void norm_scale(const float* s_sq, int st, int vq, int n,
                                            const float* s_tail, float eps, float* s_part,
-                                           float* s_scale) {
+                                           float* s_scale, int tid = threadIdx.x) {
 #pragma clang fp contract(off)
     static_assert(T % 4 == 0 && T >= 8, "T: whole float4 loads");
     constexpr int F4 = T / 4;
-    const int tid = threadIdx.x;
     if (tid < 4) {
         // two buffers of T terms take turns (no register copies between
         // the dependent adds): one is added while the other is read
