@@ -35,9 +35,11 @@
 // by DMA, so no registers are held for it.  With 80 KiB of LDS (KSP 1) two
 // workgroups share a CU, and one's MFMAs run beside the other's splitting.
 //
-// Non-finite values.  inf, and finite values that round to a bf16 inf, make
-// NaN when split.  A wave whose result is not finite therefore computes its
-// rows again in plain f32 from the cache (attend_plain).
+// Values that cannot be split.  inf, and finite values that round to a bf16 inf,
+// make NaN when split, and the remainders of values below 2^-109 run out of
+// bf16's exponents.  A wave with a result that is not finite, or nonzero and
+// below 2^-100, therefore computes its rows again in plain f32 from the cache
+// (attend_plain).
 #include <math.h>
 
 #include "attn_common.h"
@@ -530,11 +532,16 @@ __global__ __launch_bounds__(64 * QS * HW * KSP, 2) void prefill_split_kernel(
     };
     float lt = rows_sum(l);
     float z = lt * 0.0f;  // NaN once any of the row's values is not finite
+    unsigned least = ~0u;  // magnitude bits of the least nonzero value, times two, less one
 #pragma unroll
     for (int i = 0; i < NDT; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) z = fmaf(o[i][r], 0.0f, z);
-    if (__any(row_ok && z != z)) {
+        for (int r = 0; r < 4; ++r) {
+            z = fmaf(o[i][r], 0.0f, z);
+            least = min(least, (__float_as_uint(o[i][r]) << 1) - 1u);
+        }
+    constexpr unsigned kLeast = ((127u - 100u) << 24) - 1u;  // of 2^-100
+    if (__any(row_ok && (z != z || least < kLeast))) {
         reset();
 #pragma unroll 1
         for (int kb = 0; kb <= wave_last_pos; kb += KT) attend_plain(kb);

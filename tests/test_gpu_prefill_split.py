@@ -111,3 +111,21 @@ def test_values_that_cannot_be_split(hd, heads, kvh, start, n):
     ok[np.ix_(pos >= j_v, cols0 + 3)] = False
     ok[np.ix_(pos >= j_big, cols0 + 5)] = False
     assert (np.abs(got - ref)[ok] <= 2e-5 * np.maximum(mag, 1e-3)[ok]).all()
+
+
+@pytest.mark.parametrize("hd,heads,kvh,start,n", [(128, 2, 1, 100, 60), (128, 32, 8, 0, 600),
+                                                  (64, 32, 8, 0, 500)])
+def test_small_values(hd, heads, kvh, start, n):
+    """V so small that its remainders lie below the least bf16."""
+    rows = start + n
+    q = gen([77, n], (n, heads * hd))
+    k = gen([78, n], (rows, kvh * hd))
+    v = gen([79, n], (rows, kvh * hd)) * np.float32(2.0 ** -122)
+    v[:, 1] = 0
+    ref, mag, smax = attend64(heads, kvh, start, q, k, v)
+    got = run(heads, kvh, start, q, k, v)
+    assert (got[:, 1] == 0).all()
+    # Roundings of 2^-24: one per key in the output and row sums, per score hd/4
+    # + 2 accumulations; and of 2^-150, the least f32's half, one per key.
+    bound = (2 * rows + 2 * (hd / 4 + 3) * 1.4427 * smax + 16) * 2.0 ** -24
+    assert (np.abs(got - ref) <= bound * mag + rows * 2.0 ** -150).all()
