@@ -73,6 +73,36 @@ __device__ __forceinline__ void store_q8_quad(const Q8Out& o, long row, int blk,
     }
 }
 
+// Quantizes block blk of row `row` from lanes l and l + 32 of a wave (value 4a +
+// b of half h: element 8a + 4h + b, a 32x32 MFMA's rows) and, with ok (the same
+// in both lanes), stores it without its sum, 16 bytes from each half.  All
+// lanes must be active.
+__device__ __forceinline__ void store_q8_halves(const Q8Out& o, long row, int blk, int half,
+                                                const float (&v)[16], bool ok) {
+#pragma clang fp contract(off)
+    float amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const float av = fabsf(v[i]);
+        amax = av > amax ? av : amax;
+    }
+    const float other = __shfl_xor(amax, 32);
+    amax = other > amax ? other : amax;
+    const float d = amax / 127.0f;
+    const float id = amax != 0.0f ? 127.0f / amax : 0.0f;
+    uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+        w[i >> 2] |= (uint32_t)(q8_value(v[i] * id) & 0xFF) << (8 * (i & 3));
+    // dwords 2a + h -> 4h .. 4h + 3
+    const auto lo = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
+    if (!ok) return;
+    *reinterpret_cast<uint4*>(o.q + (row * o.nb + blk) * 8 + 4 * half) =
+        make_uint4(lo[0], lo[1], hi[0], hi[1]);
+    if (half == 0) o.d[row * o.d_stride + blk] = h2f(f2h(d));
+}
+
 // sample_argmax's order (transformer.rs:654-666) for a parallel scan: the
 // larger value wins, a tie goes to the lower index; i < 0 marks "none".
 __device__ __forceinline__ void argmax_merge(float& v, int& i, float v2, int i2) {

@@ -710,6 +710,7 @@ struct GemmParams {
     int nb;
     int d_stride;          // nb rounded up to 8 (weights and activations alike)
     int batch;
+    Q8Out act;             // with ACT: silu(m[0] . x) * (m[1] . x) as Q8_0 blocks
 };
 
 constexpr int kScaleChunk = 8;  // blocks whose scales one 128-bit load covers
@@ -764,7 +765,18 @@ __device__ __forceinline__ float sum_f32(int d) {
     return SUB ? __int_as_float(d) - kSumBase : (float)d;
 }
 
-template <int WRW, int WTW, int NTS>
+// With ACT the two matrices are gate and up of a block: a workgroup's rows are
+// the same 32 hidden rows of gate and of up in turn, a gate and an up wave swap
+// half their tokens through LDS, and each writes SwiGLU's 32 values per token
+// as one Q8_0 block, the input of the down projection.  The f32 rows
+// (operations and order as swiglu_kernel's) never go to memory: 2048 tokens of
+// hidden 14336 write 33 MB instead of 235 MB that a second launch read back.
+// A whole layer's prefill, separate launches -> this: dim 4096, hidden 14336,
+// 512 / 1024 / 2048 / 4096 tokens 579 -> 574, 1012 -> 955, 1990 -> 1950, 4480 ->
+// 4330 us; dim 576, hidden 1536, 130 / 512 tokens 56 -> 53, 73 -> 70; dim 288,
+// hidden 768, 300 tokens 52 -> 47.  (The exp's VALU work in the epilogue takes
+// back about half of what the memory traffic cost.)
+template <int WRW, int WTW, int NTS, bool ACT>
 __global__ __launch_bounds__(64 * WRW * WTW) void gemm_q4_mfma_kernel(GemmParams p) {
 #pragma clang fp contract(off)
     using Sh = GemmShape<WRW, WTW, NTS>;
@@ -788,8 +800,12 @@ __global__ __launch_bounds__(64 * WRW * WTW) void gemm_q4_mfma_kernel(GemmParams
     const QMat M = m == 0 ? p.m[0] : (m == 1 ? p.m[1] : p.m[2]);
     const int nb = p.nb;
     const int ds = p.d_stride;
-    const int wr0 = rt * RT;  // workgroup's first row / token
+    const int wr0 = rt * (ACT ? RT / 2 : RT);  // workgroup's first row / token
     const int wt0 = tt * TT;
+    // row of the matrix (with ACT: of gate or up, by bit 5) at tile row r
+    auto mat_row = [&](int r) {
+        return min(wr0 + (ACT ? (r >> 6 << 5) + (r & 31) : r), M.rows - 1);
+    };
 
     // Stage loads, all 16 bytes wide and coalesced, addresses clamped into
     // the buffers (rows / tokens / blocks past the end are never used):
@@ -798,9 +814,12 @@ __global__ __launch_bounds__(64 * WRW * WTW) void gemm_q4_mfma_kernel(GemmParams
     //   weight scales: threads 0..RT-1 -> row; activation scales: the next
     //   2*TT threads, half a token's eight each.
     const int lrow = tid >> 2, lsub = tid & 3;
-    const uint8_t* asrc = M.qs + (long)min(wr0 + lrow, M.rows - 1) * nb * 16;
+    const int drow = min(tid, RT - 1);
+    const uint8_t* aqs = ACT && (lrow & 32) ? p.m[1].qs : M.qs;
+    const uint16_t* adw = ACT && (drow & 32) ? p.m[1].d : M.d;
+    const uint8_t* asrc = aqs + (long)mat_row(lrow) * nb * 16;
     const uint32_t* bsrc = p.aq + (long)min(wt0 + lrow, p.batch - 1) * nb * 8;
-    const uint16_t* dwsrc = M.d + (long)min(wr0 + min(tid, RT - 1), M.rows - 1) * ds;
+    const uint16_t* dwsrc = adw + (long)mat_row(drow) * ds;
     const int sidx = min(max(tid - RT, 0), 2 * TT - 1);
     const float* dasrc = p.ad + (long)min(wt0 + (sidx >> 1), p.batch - 1) * ds + 4 * (sidx & 1);
     uint4 ra0, ra1, rb0, rb1, rb2, rb3, rs;
@@ -917,6 +936,37 @@ __global__ __launch_bounds__(64 * WRW * WTW) void gemm_q4_mfma_kernel(GemmParams
                 }
         }
         if (sg + 1 < n_stages) SLM_GEMM_STORE_STAGE(st[(sg + 1) & 1]);
+    }
+
+    if constexpr (ACT) {
+        // wave 2i (gate) keeps its first 32 tokens and hands over the others,
+        // wave 2i + 1 (up) the reverse; with 32 tokens the gate wave takes all
+        const bool up = wave & 1;
+        float* x = reinterpret_cast<float*>(&st[0]) + lane;
+        __syncthreads();  // the stages have been read
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+            if (NTS > 1 || up) {
+                // values: a choice between the elements themselves would put
+                // the accumulators into scratch memory
+                const float first = acc[0][j], last = acc[NTS - 1][j];
+                x[1024 * wave + 64 * j] = up ? first : last;
+            }
+        __syncthreads();
+        if (NTS == 1 && up) return;
+        float y[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const float got = x[1024 * (wave ^ 1) + 64 * j];
+            const float first = acc[0][j], last = acc[NTS - 1][j];
+            const float g = up ? got : first;
+            const float u = up ? last : got;
+            y[j] = jit_silu(g) * u;
+        }
+        const int t = wt0 + qt + (up ? 32 : 0) + l32;
+        const int h0 = wr0 + (qr >> 6 << 5);
+        store_q8_halves(p.act, t, h0 >> 5, hh, y, t < p.batch && h0 < M.rows);
+        return;
     }
 
     // Rows r0..r0+3 of token t (r0 a multiple of 4) are contiguous in out and
@@ -1306,7 +1356,24 @@ hipError_t launch_gemm_t(const Q4Job* jobs, int njobs, const uint32_t* aq, const
     GemmParams p;
     const unsigned grid = gemm_params(jobs, njobs, aq, ad, nb, batch, Sh::RT, Sh::TT, &p);
     if (!grid) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((gemm_q4_mfma_kernel<WRW, WTW, NTS>), dim3(grid), dim3(Sh::NT), 0, st, p);
+    hipLaunchKernelGGL((gemm_q4_mfma_kernel<WRW, WTW, NTS, false>), dim3(grid), dim3(Sh::NT), 0,
+                       st, p);
+    return hipGetLastError();
+}
+
+template <int WRW, int WTW, int NTS>
+hipError_t launch_gemm_swiglu_t(const Q4Job& gate, const Q4Job& up, const uint32_t* aq,
+                                const float* ad, int nb, int batch, const Q8Out& act,
+                                hipStream_t st) {
+    using Sh = GemmShape<WRW, WTW, NTS>;
+    GemmParams p;
+    // one pass over gate's rows, half a tile of them (and the same of up) per workgroup
+    const unsigned grid = gemm_params(&gate, 1, aq, ad, nb, batch, Sh::RT / 2, Sh::TT, &p);
+    if (!grid) return hipErrorInvalidValue;
+    p.m[1] = QMat{up.qs, up.d, up.out, up.res, up.rows, up.out_stride, q4_scale_stride(nb)};
+    p.act = act;
+    hipLaunchKernelGGL((gemm_q4_mfma_kernel<WRW, WTW, NTS, true>), dim3(grid), dim3(Sh::NT), 0,
+                       st, p);
     return hipGetLastError();
 }
 
@@ -1392,8 +1459,6 @@ long device_cus() {
     return n;
 }
 
-}  // namespace
-
 // Tile choice.  Up to four 16 x 16 workgroups per CU the blocks are split over
 // the waves (gemm_q4_small_kernel): its time grows with the workgroups (25 ns
 // each at 128 blocks, beside a floor of about 8 us), that of the tiles below
@@ -1412,9 +1477,9 @@ long device_cus() {
 // would leave CUs idle (Wo at 512 tokens: 128 workgroups of 128 x 128 on 256
 // CUs).  Tile shape does not change results (each output is one thread's
 // ordered sum over blocks).
-hipError_t launch_q4_gemm(const Q4Job* jobs, int njobs, const uint32_t* aq, const float* ad,
-                          int nb, int batch, hipStream_t st) {
-    if (njobs < 1 || njobs > 3 || batch < 1) return hipErrorInvalidValue;
+enum class GemmForm { kSmall, k64, k128 };
+
+GemmForm gemm_form(const Q4Job* jobs, int njobs, int batch) {
     long w128 = 0, w64 = 0, w16 = 0;
     for (int i = 0; i < njobs; ++i) {
         w128 += (long)((jobs[i].rows + 127) / 128) * ((batch + 127) / 128);
@@ -1423,11 +1488,39 @@ hipError_t launch_q4_gemm(const Q4Job* jobs, int njobs, const uint32_t* aq, cons
                ((batch + kSmallToks - 1) / kSmallToks);
     }
     const long cus = device_cus();
+    if (w16 <= 4 * cus) return GemmForm::kSmall;
     const double t128 = (double)((w128 + cus - 1) / cus) * 4.0;
     const double t64 = (double)((w64 + cus - 1) / cus) * 1.1;
-    if (w16 <= 4 * cus) return launch_gemm_small(jobs, njobs, aq, ad, nb, batch, st);
-    return t128 < t64 ? launch_gemm_t<4, 2, 2>(jobs, njobs, aq, ad, nb, batch, st)
-                      : launch_gemm_t<2, 2, 1>(jobs, njobs, aq, ad, nb, batch, st);
+    return t128 < t64 ? GemmForm::k128 : GemmForm::k64;
+}
+
+}  // namespace
+
+hipError_t launch_q4_gemm(const Q4Job* jobs, int njobs, const uint32_t* aq, const float* ad,
+                          int nb, int batch, hipStream_t st) {
+    if (njobs < 1 || njobs > 3 || batch < 1) return hipErrorInvalidValue;
+    switch (gemm_form(jobs, njobs, batch)) {
+        case GemmForm::kSmall: return launch_gemm_small(jobs, njobs, aq, ad, nb, batch, st);
+        case GemmForm::k128: return launch_gemm_t<4, 2, 2>(jobs, njobs, aq, ad, nb, batch, st);
+        case GemmForm::k64: break;
+    }
+    return launch_gemm_t<2, 2, 1>(jobs, njobs, aq, ad, nb, batch, st);
+}
+
+bool q4_gemm_takes_swiglu(const Q4Job& gate, const Q4Job& up, int batch) {
+    const Q4Job jobs[2] = {gate, up};
+    return gate.rows == up.rows && gate.rows % 32 == 0 && batch >= 1 &&
+           gemm_form(jobs, 2, batch) != GemmForm::kSmall;
+}
+
+hipError_t launch_q4_gemm_swiglu(const Q4Job& gate, const Q4Job& up, const uint32_t* aq,
+                                 const float* ad, int nb, int batch, const Q8Out& act,
+                                 hipStream_t st) {
+    if (!q4_gemm_takes_swiglu(gate, up, batch)) return hipErrorInvalidValue;
+    const Q4Job jobs[2] = {gate, up};
+    return gemm_form(jobs, 2, batch) == GemmForm::k128
+               ? launch_gemm_swiglu_t<4, 2, 2>(gate, up, aq, ad, nb, batch, act, st)
+               : launch_gemm_swiglu_t<2, 2, 1>(gate, up, aq, ad, nb, batch, act, st);
 }
 
 }  // namespace slm

@@ -154,6 +154,13 @@ hipError_t launch_q4_gemv_norm_swiglu(const Q4Job& gate, const Q4Job& up, const 
 // any batch, from pre-quantized activations
 hipError_t launch_q4_gemm(const Q4Job* jobs, int njobs, const uint32_t* aq, const float* ad,
                           int nb, int batch, hipStream_t st);
+// gate and up with SwiGLU fused: Q8_0 blocks of silu(gate . x) * (up . x), no
+// block sums; for the batches that q4_gemm_takes_swiglu names (the others have
+// so few tiles that the separate launches' split over the blocks is faster)
+bool q4_gemm_takes_swiglu(const Q4Job& gate, const Q4Job& up, int batch);
+hipError_t launch_q4_gemm_swiglu(const Q4Job& gate, const Q4Job& up, const uint32_t* aq,
+                                 const float* ad, int nb, int batch, const Q8Out& act,
+                                 hipStream_t st);
 
 // JIT kernels (norm_act.hip).  RMSNorm (w != nullptr) or L2 norm (w ==
 // nullptr) of `rows` rows of n, into out (f32) and/or q8 (n % 32 == 0).

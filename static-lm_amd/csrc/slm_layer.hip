@@ -204,26 +204,33 @@ int slm_layer_forward_dev(slm_attn_ctx* c, int32_t layer, int32_t start, int32_t
         t.done();
         if ((rc = run(c, e, "rmsnorm kernel launch"))) return rc;
     }
-    // gate and up (:617-636)
-    {
-        const slm::Q4Job jobs[2] = {q4_job(w->w_gate, hb), q4_job(w->w_up, hb2)};
+    // gate and up (:617-636), then SwiGLU straight to Q8_0 (:638): in the
+    // projection itself, whose blocks then lie in the hidden rows' buffer
+    // (its input is still being read), or in a launch of its own
+    slm::Q8Out act = q8_out(c, nbh);
+    const slm::Q4Job gate = q4_job(w->w_gate, hb), up = q4_job(w->w_up, hb2);
+    if (slm::q4_gemm_takes_swiglu(gate, up, n)) {
+        act.q = reinterpret_cast<uint32_t*>(hb);  // n * hidden bytes
+        act.d = hb2;  // n * d_stride floats, at most n * hidden
+        Timed t(c, SLM_K_GEMM);
+        hipError_t e = slm::launch_q4_gemm_swiglu(gate, up, c->q8_q, c->q8_d, nb, n, act, st);
+        t.done();
+        if ((rc = run(c, e, "q4 projection kernel launch"))) return rc;
+    } else {
+        const slm::Q4Job jobs[2] = {gate, up};
         Timed t(c, SLM_K_GEMM);
         hipError_t e = slm::launch_q4_gemm(jobs, 2, c->q8_q, c->q8_d, nb, n, st);
         t.done();
         if ((rc = run(c, e, "q4 projection kernel launch"))) return rc;
-    }
-    // SwiGLU straight to Q8_0 (:638)
-    {
-        Timed t(c, SLM_K_ELEM);
-        hipError_t e = slm::launch_swiglu(hb, hb2, (long)n * hidden, hidden, nullptr,
-                                          q8_out(c, nbh), st);
-        t.done();
+        Timed ts(c, SLM_K_ELEM);
+        e = slm::launch_swiglu(hb, hb2, (long)n * hidden, hidden, nullptr, act, st);
+        ts.done();
         if ((rc = run(c, e, "swiglu kernel launch"))) return rc;
     }
     // x = x_mid + W_down . act (:640-650)
     const slm::Q4Job job = q4_job(w->w_down, x, x_mid);
     Timed t(c, SLM_K_GEMM);
-    hipError_t e = slm::launch_q4_gemm(&job, 1, c->q8_q, c->q8_d, nbh, n, st);
+    hipError_t e = slm::launch_q4_gemm(&job, 1, act.q, act.d, nbh, n, st);
     t.done();
     return run(c, e, "q4 projection kernel launch");
 }
