@@ -230,13 +230,15 @@ __global__ __launch_bounds__(64 * QS * HW * KSP, 2) void prefill_split_kernel(
             // inline assembly: the compiler must not make LDS reads of the
             // planes wait for it; the wave waits (vmcnt) before it reads its
             // share back.  M0 holds the wave's LDS destination; lane l's 16
-            // bytes land at M0 + 16*l.
+            // bytes land at M0 + 16*l.  The load must not issue in the cycle
+            // after the scalar write of M0 (one wait state, which the compiler
+            // does not put in ahead of inline assembly).
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const unsigned dst = (unsigned)(unsigned long)(
                     __attribute__((address_space(3))) float*)&sm.raw[u * 8 + h * 256];
-                asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off[i][h]), "s"(r),
-                             "{m0}"(dst) : "memory");
+                asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off[i][h]),
+                             "s"(r), "{m0}"(dst) : "memory");
             }
         }
     };
