@@ -37,11 +37,13 @@
 //
 // Values that cannot be split.  inf, and finite values that round to a bf16 inf,
 // make NaN when split, and the remainders of values below 2^-109 run out of
-// bf16's exponents.  A wave with a result that is not finite, or nonzero and
-// below 2^-100, therefore computes its rows again in f32 from the cache
-// (attend_f32, attend_plain): 4096 rows of the Llama-3-8B shape 0.87 ms per
-// call, 1.26 with one inf near the end, 2.5 with every value NaN (39 with a key
-// at a time throughout).
+// bf16's exponents.  The splitting therefore keeps the largest magnitudes of q,
+// K and V, and a wave computes its rows again in f32 from the cache
+// (attend_f32, attend_plain) if a result is not finite, q or K reach 2^64, or
+// an output sum is so small beside V's values that bits lost in P or V could
+// show (least_sum).  Looking costs 1-2% (Llama-3-8B shape, per call: 4096 rows
+// 680 -> 689 us, 777 rows at start 1000 96.7 -> 98.7), computing again several
+// times the call.
 #include <math.h>
 
 #include "attn_common.h"
@@ -74,6 +76,24 @@ struct SplitParams {
     float scale_log2;
 };
 
+// The larger one, or NaN if either is (v_maximum3_f32 for two in turn).
+__device__ __forceinline__ float maximum(float a, float b) {
+    return __builtin_elementwise_maximum(a, b);
+}
+
+// ... over the wave.
+__device__ __forceinline__ float wave_maximum(float x) {
+    x = maximum(x, dpp<0x128>(x));
+    x = maximum(x, dpp<0x124>(x));
+    x = maximum(x, dpp<0x122>(x));
+    x = maximum(x, dpp<0x121>(x));
+    const uint32_t u = __float_as_uint(x);
+    const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    const uint32_t w = __float_as_uint(maximum(__uint_as_float(a[0]), __uint_as_float(a[1])));
+    const auto b = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+    return maximum(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
 __device__ __forceinline__ v4f mfma(bf8 a, bf8 b, v4f c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
@@ -102,7 +122,7 @@ __device__ __forceinline__ void split8(const float (&x)[8], uint4 (&p)[3]) {
 }
 
 template <int HD, int HW, int QS, int KSP, bool PAIR>
-__global__ __launch_bounds__(64 * QS * HW * KSP, 2) void prefill_split_kernel(
+__global__ __launch_bounds__(64 * QS * HW * KSP, HD == 64 ? 4 : 2) void prefill_split_kernel(
     SplitParams p) {
     constexpr int NB = KSP == 1 ? 2 : 1;  // plane buffers
     
@@ -242,6 +262,16 @@ __global__ __launch_bounds__(64 * QS * HW * KSP, 2) void prefill_split_kernel(
             }
         }
     };
+    // Largest magnitudes of the K values and of the V values that this thread
+    // splits; the V values are all of dim tid % HD.
+    float top_k = 0.0f, top_v = 0.0f;
+    static_assert(NT % HD == 0 && PL % HD == 0, "a thread's V chunks share their dim");
+    auto top8 = [](float t, const float (&x)[8]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) t = maximum(maximum(t, fabsf(x[j])), fabsf(x[j + 1]));
+        asm volatile("" : "+v"(t));  // here, not after the loop's other shares: registers
+        return t;
+    };
     // Splits this wave's share into the planes of buffer buf.
     auto stage = [&](int buf) __attribute__((always_inline)) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -255,12 +285,14 @@ __global__ __launch_bounds__(64 * QS * HW * KSP, 2) void prefill_split_kernel(
                 const float4 a = ld4(&sm.raw[(u + lane) * 8]), b = ld4(&sm.raw[(u + lane) * 8 + 4]);
                 x[0] = a.x, x[1] = a.y, x[2] = a.z, x[3] = a.w;
                 x[4] = b.x, x[5] = b.y, x[6] = b.z, x[7] = b.w;
+                top_k = top8(top_k, x);
                 split8(x, pl);
 #pragma unroll
                 for (int k = 0; k < 3; ++k) sm.k[slot][k][k_slot(f / KC, f % KC)] = pl[k];
             } else {
 #pragma unroll
                 for (int j = 0; j < 8; ++j) x[j] = sm.raw[u * 8 + j * 64 + lane];
+                top_v = top8(top_v, x);
                 split8(x, pl);
                 const int d = f % HD;
 #pragma unroll
@@ -278,6 +310,7 @@ __global__ __launch_bounds__(64 * QS * HW * KSP, 2) void prefill_split_kernel(
         float x[8];
         uint4 pl[3];
         load_q8(ks, x);
+        top_k = top8(top_k, x);
         split8(x, pl);
 #pragma unroll
         for (int k = 0; k < 3; ++k) qf[k][ks] = __builtin_bit_cast(bf8, pl[k]);
@@ -446,12 +479,23 @@ __global__ __launch_bounds__(64 * QS * HW * KSP, 2) void prefill_split_kernel(
         }
     }
 
+    // For the check of the results below: every thread's top_v and each wave's
+    // largest of both, in raw bytes of the wave's own (it has read them back).
+    constexpr int kWaveRaw = 512;  // floats of a wave's chunks of share 0
+    {
+        float* t = &sm.raw[wave * kWaveRaw];
+        t[lane] = top_v;
+        t[64] = wave_maximum(top_k);  // the same in every lane
+        t[65] = wave_maximum(top_v);
+    }
+    if constexpr (KSP == 1) __syncthreads();
+
     if constexpr (KSP > 1) {
         // Merge of the key splits: splits 1..KSP-1 hand each lane's O
         // registers, max and sum partial to split 0 through LDS (lane
         // contiguous), which folds them in split order.
         constexpr int NR = NDT * 4 + 2;  // floats per lane
-        static_assert((KSP - 1) * NWS * 64 * NR * 4 <= (int)sizeof(sm), "the merge fits the LDS");
+        static_assert((KSP - 1) * NWS * 64 * NR * 4 <= (int)sizeof(sm.k), "clear of raw");
         float* s_merge = reinterpret_cast<float*>(&sm);
         const int ws = qs * HW + hw;
         if (kspl > 0) {
@@ -558,18 +602,51 @@ __global__ __launch_bounds__(64 * QS * HW * KSP, 2) void prefill_split_kernel(
             }
         }
     };
+    // Where the planes may not hold enough of an operand (bf16's exponents end
+    // at 2^-126, and planes below that may count as zero): with kv_len keys,
+    // probabilities up to 2^kLazyRescale and values up to top, an output sum is
+    // off by less than kv_len * (top + 2^kLazyRescale) * 2^-122, which is in
+    // f32's last bits of a sum of at least least_sum(top); a score of operands
+    // below 2^64 by less than 2^-50.
     float lt = rows_sum(l);
+    auto least_sum = [&](float top) {
+        return (float)kv_len * fmaf(top, 0x1p-96f, 0x1p-96f * (1 << (int)kLazyRescale));
+    };
     float z = lt * 0.0f;  // NaN once any of the row's values is not finite
-    unsigned least = ~0u;  // magnitude bits of the least nonzero value, times two, less one
+    float least = INFINITY;
 #pragma unroll
     for (int i = 0; i < NDT; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             z = fmaf(o[i][r], 0.0f, z);
-            least = min(least, (__float_as_uint(o[i][r]) << 1) - 1u);
+            least = fminf(least, fabsf(o[i][r]));
         }
-    constexpr unsigned kLeast = ((127u - 100u) << 24) - 1u;  // of 2^-100
-    if (__any(row_ok && (z != z || least < kLeast))) {
+    top_k = top_v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        top_k = maximum(top_k, sm.raw[w * kWaveRaw + 64]);
+        top_v = maximum(top_v, sm.raw[w * kWaveRaw + 65]);
+    }
+    bool again = z != z || !(top_k < 0x1p64f);
+    if (!again && !(least >= least_sum(top_v))) {
+        // by dim: a dim whose values are all zero has a sum of zero
+#pragma unroll
+        for (int i = 0; i < NDT; ++i) {
+            const int d = 16 * i + 4 * lg;
+            float t[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+            for (int j = 0; j < NT / HD; ++j) {
+                const int at = j * HD + d;
+                const float4 x = ld4(&sm.raw[(at >> 6) * kWaveRaw + (at & 63)]);
+                t[0] = maximum(t[0], x.x), t[1] = maximum(t[1], x.y);
+                t[2] = maximum(t[2], x.z), t[3] = maximum(t[3], x.w);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                again |= t[r] != 0.0f && !(fabsf(o[i][r]) >= least_sum(t[r]));
+        }
+    }
+    if (__any(row_ok && again)) {
         reset();
         float x[NKS][8];
 #pragma unroll

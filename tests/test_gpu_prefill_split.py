@@ -129,3 +129,64 @@ def test_small_values(hd, heads, kvh, start, n):
     # + 2 accumulations; and of 2^-150, the least f32's half, one per key.
     bound = (2 * rows + 2 * (hd / 4 + 3) * 1.4427 * smax + 16) * 2.0 ** -24
     assert (np.abs(got - ref) <= bound * mag + rows * 2.0 ** -150).all()
+
+
+RANGE_CASES = [(128, 2, 1, 100, 60), (128, 32, 8, 0, 600), (128, 32, 32, 0, 1100),
+               (64, 32, 8, 0, 500), (64, 32, 8, 3, 1300)]
+
+
+@pytest.mark.parametrize("expo", [-120, 120])
+@pytest.mark.parametrize("hd,heads,kvh,start,n", RANGE_CASES)
+def test_scores_of_tiny_and_huge_operands(hd, heads, kvh, start, n, expo):
+    """Ordinary scores of a q whose remainders lie below the least bf16 with a
+    k that makes up for it, and the other way round."""
+    rows = start + n
+    q = gen([80, n], (n, heads * hd)) * np.float32(2.0 ** expo)
+    k = gen([81, n], (rows, kvh * hd)) * np.float32(2.0 ** -expo)
+    v = gen([82, n], (rows, kvh * hd))
+    ref, mag, smax = attend64(heads, kvh, start, q, k, v)
+    got = run(heads, kvh, start, q, k, v)
+    # Roundings of 2^-24: one per key in the output and row sums, per score hd/4
+    # + 3; and of q, pre-scaled, to a multiple of 2^-149.
+    bound = (2 * rows + 2 * (hd / 4 + 3) * 1.4427 * smax + 16 + 64) * 2.0 ** -24
+    assert (np.abs(got - ref) <= bound * mag).all(), (np.abs(got - ref) / mag).max() / bound
+
+
+@pytest.mark.parametrize("hd,heads,kvh,start,n", RANGE_CASES)
+def test_tiny_probabilities_of_huge_values(hd, heads, kvh, start, n):
+    """Key 0 has all the weight but only zero values: what counts are the other
+    keys' probabilities of 2^-125 to 2^-124."""
+    rows = start + n
+    scale = np.float32(1.4426950408889634) / np.sqrt(np.float32(hd))
+    one = np.float32(1) / scale
+    one = next(x for x in (one, np.nextafter(one, np.float32(0)), np.nextafter(one, np.float32(99)))
+               if x * scale == 1)  # scores in log2 units are then k's first dim, exactly
+    q = np.zeros((n, heads * hd), np.float32)
+    q[:, ::hd] = one
+    k = np.zeros((rows, kvh * hd), np.float32)
+    k[1:, ::hd] = np.floor(np.abs(gen([83, n], (rows - 1, kvh))) * 64) % 64 / 64 - 125
+    v = gen([84, n], (rows, kvh * hd)) * np.float32(2.0 ** 120)
+    v[0] = 0
+    ref, mag, _ = attend64(heads, kvh, start, np.where(q != 0, np.sqrt(hd) * np.log(2), 0.0), k, v)
+    got = run(heads, kvh, start, q, k, v)
+    # Roundings of 2^-24: one per key in the output and row sums, and a few in
+    # exp2 and the normalisation.
+    bound = (2 * rows + 16) * 2.0 ** -24
+    assert (np.abs(got - ref) <= bound * mag).all()
+
+
+@pytest.mark.parametrize("hd,heads,kvh,start,n", RANGE_CASES)
+def test_values_below_the_least_bf16(hd, heads, kvh, start, n):
+    """Values that bf16 rounds to zero, in some dims; the other dims hold zeros
+    and ordinary values."""
+    rows = start + n
+    q = gen([85, n], (n, heads * hd))
+    k = gen([86, n], (rows, kvh * hd))
+    v = gen([87, n], (rows, kvh * hd))
+    v[:, 1::3] *= np.float32(2.0 ** -138)
+    v[:, 2::3] = 0
+    ref, mag, smax = attend64(heads, kvh, start, q, k, v)
+    got = run(heads, kvh, start, q, k, v)
+    # as test_small_values
+    bound = (2 * rows + 2 * (hd / 4 + 3) * 1.4427 * smax + 16) * 2.0 ** -24
+    assert (np.abs(got - ref) <= bound * mag + rows * 2.0 ** -150).all()
