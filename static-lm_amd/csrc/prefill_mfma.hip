@@ -654,10 +654,11 @@ hipError_t launch_hd(const Shape& s, const PrefillParams& pp, hipStream_t st) {
         case PrefillKernel::kPairedFourHeads:
             if constexpr (HD <= 96) return launch_t<HD, 4, 2, 1, true>(s, pp, st);
             break;
+        // hd 128: prefill_split_plan() takes these but for batches of many
+        // heads that end before row 128
         case PrefillKernel::kDma:
-        case PrefillKernel::kDmaPaired:
-        case PrefillKernel::kPairedTwoHeads:
-            break;  // hd 128: prefill_split_plan() takes these
+        case PrefillKernel::kDmaPaired: return launch_t<HD, 4, 1, 1>(s, pp, st);
+        case PrefillKernel::kPairedTwoHeads: return launch_t<HD, 2, 2, 1>(s, pp, st);
         case PrefillKernel::kPairedOneHead:
             if constexpr (HD == 128) return launch_t<128, 1, 2, 4, true>(s, pp, st);
             break;

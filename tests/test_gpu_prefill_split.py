@@ -78,6 +78,13 @@ def test_against_float64(hd, heads, kvh, start, n):
     assert rel < 3e-6, rel
 
 
+@pytest.mark.parametrize("start,n", [(0, 97), (0, 127), (30, 97)])
+def test_many_heads_before_row_128(start, n):
+    """Batches too short for the split kernel with so many heads that they fill
+    the CUs several times over."""
+    test_against_float64(128, 1024, 64, start, n)
+
+
 @pytest.mark.parametrize("hd,heads,kvh,start,n", [(128, 2, 1, 100, 60), (128, 32, 8, 0, 600),
                                                   (128, 32, 32, 0, 1100), (64, 32, 8, 0, 500)])
 def test_values_that_cannot_be_split(hd, heads, kvh, start, n):
