@@ -238,29 +238,30 @@ int slm_attn_profile_read(slm_attn_ctx* ctx, slm_kernel_stat* out /* [SLM_K_COUN
 int slm_attn_decode_splits(const slm_attn_ctx* ctx, int32_t seq_len,
                            int32_t* n_splits, int32_t* tile);
 
-/* The tiling of a causal prefill of n rows from row start (slm_attn_prefill,
+/* The kernel a causal prefill of n rows from row start runs (slm_attn_prefill,
  * slm_attn_prefill_dev and the blocks built on them).  Like the decode split
  * layout, a pure function of start, n, the config and the device's CU count;
  * no counterpart in the reference, which has one scalar path: it is for tests
- * and benchmarks that need to know which batches run alike.  Heads per
- * workgroup are query heads of one KV head; query blocks are 16 rows;
- * "paired" workgroups take blocks i and n_blocks-1-i, so every workgroup has
- * the same causal work.  The tilings are those of the f32 matrix kernels; most
- * larger batches of head_dim 64 and 128 run instead on bf16 matrix cores with
- * f32 operands split in three, eight waves of one head and block (or half a
- * block's keys) per workgroup.  SLM_ERR_BATCH as slm_attn_prefill for
- * an empty or out-of-range batch. */
+ * and benchmarks that need to know which kernel ran.  Heads per workgroup are
+ * query heads of one KV head; query blocks are 16 rows; "paired" workgroups
+ * take blocks i and n_blocks-1-i, so every workgroup has the same causal
+ * work.  The SPLIT forms run on bf16 matrix cores with f32 operands split in
+ * three, eight waves of one head and block (and key split) per workgroup; the
+ * others on f32 ones.  (A batch of one row runs the decode kernel, whatever
+ * this names.)  SLM_ERR_BATCH as slm_attn_prefill for an empty or
+ * out-of-range batch. */
 enum {
     SLM_PF_FOUR_HEADS = 0,        /* four heads, one block (kv_mul % 4 == 0) */
     SLM_PF_THREE_HEADS = 1,       /* three heads, one block (kv_mul % 3 == 0) */
     SLM_PF_TWO_HEADS = 2,         /* two heads, two blocks (kv_mul even) */
     SLM_PF_ONE_HEAD = 3,          /* one head, four blocks */
     SLM_PF_KEY_SPLIT = 4,         /* one head, one block, key tiles over four waves (hd <= 64) */
-    SLM_PF_PAIRED_FOUR_HEADS = 5, /* four heads, paired blocks (hd <= 96) */
-    SLM_PF_DMA = 6,               /* hd 128, from 4 workgroups per CU: four heads, two blocks */
-    SLM_PF_DMA_PAIRED = 7,        /* hd 128, a whole number per CU: the same, paired blocks */
-    SLM_PF_PAIRED_TWO_HEADS = 8,  /* hd 128: two heads, paired blocks, two key splits */
-    SLM_PF_PAIRED_ONE_HEAD = 9    /* hd 128: one head, paired blocks, four key splits */
+    SLM_PF_PAIRED_FOUR_HEADS = 5, /* four heads, paired blocks (hd 16, 32, 48, 96) */
+    /* 6 to 8: kernels that are gone */
+    SLM_PF_PAIRED_ONE_HEAD = 9,   /* hd 128: one head, paired blocks, four key splits */
+    SLM_PF_SPLIT_KEYS = 10,       /* hd 64, 128: four (head, block), paired, two key splits */
+    SLM_PF_SPLIT_PAIRED = 11,     /* hd 64, 128: eight (head, block), paired */
+    SLM_PF_SPLIT_CONSECUTIVE = 12 /* hd 64, 128: eight (head, block), consecutive blocks */
 };
 int slm_attn_prefill_kernel(const slm_attn_ctx* ctx, int32_t start, int32_t n,
                             int32_t* kernel);

@@ -67,9 +67,9 @@ GGML_F32, GGML_F16, GGML_Q4_0, GGML_Q8_0 = 0, 1, 2, 8
 KERNEL_KINDS = ("append", "decode", "combine", "prefill", "rope", "quant", "gemm", "norm",
                 "elem")
 # prefill kernels, numbered as SLM_PF_* (slm_attn_prefill_kernel)
-PREFILL_KERNELS = ("four_heads", "three_heads", "two_heads", "one_head", "key_split",
-                   "paired_four_heads", "dma", "dma_paired", "paired_two_heads",
-                   "paired_one_head")
+PREFILL_KERNELS = {0: "four_heads", 1: "three_heads", 2: "two_heads", 3: "one_head",
+                   4: "key_split", 5: "paired_four_heads", 9: "paired_one_head",
+                   10: "split_keys", 11: "split_paired", 12: "split_consecutive"}
 
 
 class SlmAttnError(RuntimeError):

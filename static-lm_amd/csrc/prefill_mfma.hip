@@ -641,9 +641,9 @@ hipError_t launch_t(const Shape& s, const PrefillParams& pp, hipStream_t st) {
 }
 
 template <int HD>
-hipError_t launch_hd(const Shape& s, const PrefillParams& pp, hipStream_t st) {
-    // (at hd 128 only what prefill_split_plan() leaves comes here)
-    switch (prefill_plan(s.head_dim, s.num_heads, s.kv_mul, s.cus, pp.start, pp.n)) {
+hipError_t launch_hd(const Shape& s, const PrefillParams& pp, PrefillKernel kernel,
+                     hipStream_t st) {
+    switch (kernel) {
         case PrefillKernel::kFourHeads: return launch_t<HD, 4, 1, 1>(s, pp, st);
         case PrefillKernel::kThreeHeads: return launch_t<HD, 3, 1, 1>(s, pp, st);
         case PrefillKernel::kTwoHeads: return launch_t<HD, 2, 2, 1>(s, pp, st);
@@ -652,16 +652,14 @@ hipError_t launch_hd(const Shape& s, const PrefillParams& pp, hipStream_t st) {
             if constexpr (HD <= 64) return launch_t<HD, 1, 1, 4>(s, pp, st);
             break;
         case PrefillKernel::kPairedFourHeads:
-            if constexpr (HD <= 96) return launch_t<HD, 4, 2, 1, true>(s, pp, st);
+            if constexpr (HD <= 96 && HD != 64) return launch_t<HD, 4, 2, 1, true>(s, pp, st);
             break;
-        // hd 128: prefill_split_plan() takes these but for batches of many
-        // heads that end before row 128
-        case PrefillKernel::kDma:
-        case PrefillKernel::kDmaPaired: return launch_t<HD, 4, 1, 1>(s, pp, st);
-        case PrefillKernel::kPairedTwoHeads: return launch_t<HD, 2, 2, 1>(s, pp, st);
         case PrefillKernel::kPairedOneHead:
             if constexpr (HD == 128) return launch_t<128, 1, 2, 4, true>(s, pp, st);
             break;
+        case PrefillKernel::kSplitKeys:
+        case PrefillKernel::kSplitPaired:
+        case PrefillKernel::kSplitConsecutive: break;  // not this kernel's
     }
     return hipErrorInvalidValue;  // a plan this head_dim has no kernel for
 }
@@ -686,17 +684,17 @@ hipError_t launch_prefill_mfma(const Shape& s, const PrefillArgs& a, hipStream_t
          !prefill_appends(s.head_dim, s.num_heads, s.kv_mul, s.cus, a.start, a.n)))
         return hipErrorInvalidValue;
     if (a.n > 65535 * 64) return hipErrorInvalidValue;
-    const PrefillSplit split =
-        prefill_split_plan(s.head_dim, s.num_heads, s.kv_mul, s.cus, a.start, a.n);
-    if (split != PrefillSplit::kNone) return launch_prefill_split(s, a, split, st);
+    const PrefillKernel kernel =
+        prefill_plan(s.head_dim, s.num_heads, s.kv_mul, s.cus, a.start, a.n);
+    if (on_split_kernel(kernel)) return launch_prefill_split(s, a, kernel, st);
     switch (s.head_dim) {
-        case 16: return launch_hd<16>(s, pp, st);
-        case 32: return launch_hd<32>(s, pp, st);
-        case 48: return launch_hd<48>(s, pp, st);
-        case 64: return launch_hd<64>(s, pp, st);
-        case 96: return launch_hd<96>(s, pp, st);
-        case 128: return launch_hd<128>(s, pp, st);
-        case 256: return launch_hd<256>(s, pp, st);
+        case 16: return launch_hd<16>(s, pp, kernel, st);
+        case 32: return launch_hd<32>(s, pp, kernel, st);
+        case 48: return launch_hd<48>(s, pp, kernel, st);
+        case 64: return launch_hd<64>(s, pp, kernel, st);
+        case 96: return launch_hd<96>(s, pp, kernel, st);
+        case 128: return launch_hd<128>(s, pp, kernel, st);
+        case 256: return launch_hd<256>(s, pp, kernel, st);
         default: return hipErrorInvalidValue;
     }
 }

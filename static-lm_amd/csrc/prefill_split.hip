@@ -679,21 +679,20 @@ hipError_t launch_t(const Shape& s, const SplitParams& pp, hipStream_t st) {
 }
 
 template <int HD, int HW>
-hipError_t launch_hw(const Shape& s, const SplitParams& pp, PrefillSplit form, hipStream_t st) {
+hipError_t launch_hw(const Shape& s, const SplitParams& pp, PrefillKernel form, hipStream_t st) {
     switch (form) {
-        case PrefillSplit::kKeySplit: return launch_t<HD, HW, 4 / HW, 2, true>(s, pp, st);
-        case PrefillSplit::kPaired: return launch_t<HD, HW, 8 / HW, 1, true>(s, pp, st);
-        case PrefillSplit::kConsecutive: return launch_t<HD, HW, 8 / HW, 1, false>(s, pp, st);
-        case PrefillSplit::kNone: break;
+        case PrefillKernel::kSplitKeys: return launch_t<HD, HW, 4 / HW, 2, true>(s, pp, st);
+        case PrefillKernel::kSplitPaired: return launch_t<HD, HW, 8 / HW, 1, true>(s, pp, st);
+        case PrefillKernel::kSplitConsecutive: return launch_t<HD, HW, 8 / HW, 1, false>(s, pp, st);
+        default: return hipErrorInvalidValue;
     }
-    return hipErrorInvalidValue;
 }
 
 template <int HD>
-hipError_t launch_hd(const Shape& s, const SplitParams& pp, PrefillSplit form, hipStream_t st) {
+hipError_t launch_hd(const Shape& s, const SplitParams& pp, PrefillKernel form, hipStream_t st) {
     // four heads on the tiles where there are so many: 4096 rows of the
     // Llama-3-8B shape 672 against 690 us with two
-    if (form == PrefillSplit::kConsecutive && s.kv_mul % 4 == 0)
+    if (form == PrefillKernel::kSplitConsecutive && s.kv_mul % 4 == 0)
         return launch_t<HD, 4, 2, 1, false>(s, pp, st);
     return s.kv_mul % 2 == 0 ? launch_hw<HD, 2>(s, pp, form, st)
                              : launch_hw<HD, 1>(s, pp, form, st);
@@ -701,7 +700,7 @@ hipError_t launch_hd(const Shape& s, const SplitParams& pp, PrefillSplit form, h
 
 }  // namespace
 
-hipError_t launch_prefill_split(const Shape& s, const PrefillArgs& a, PrefillSplit form,
+hipError_t launch_prefill_split(const Shape& s, const PrefillArgs& a, PrefillKernel form,
                                 hipStream_t st) {
     SplitParams pp{a.q,   a.k_cache, a.v_cache,   a.cos_t,  a.sin_t,  a.out, a.start,
                    a.n,   s.dim,     s.num_heads, s.kv_dim, s.kv_mul, s.half,

@@ -88,10 +88,10 @@ struct PrefillArgs {
 hipError_t launch_prefill_mfma(const Shape& s, const PrefillArgs& a,
                                hipStream_t st);
 // The same on bf16 matrix cores with f32 operands split in three
-// (prefill_split.hip), in the form that prefill_split_plan() gives;
+// (prefill_split.hip), in one of prefill_plan()'s kSplit forms;
 // launch_prefill_mfma calls it.
-enum class PrefillSplit : int;
-hipError_t launch_prefill_split(const Shape& s, const PrefillArgs& a, PrefillSplit form,
+enum class PrefillKernel : int;
+hipError_t launch_prefill_split(const Shape& s, const PrefillArgs& a, PrefillKernel form,
                                 hipStream_t st);
 
 // Q4_0 x Q8_0 projections (quant_gemm.hip).  A job is one weight matrix:

@@ -188,64 +188,66 @@ def xorshift_f32(n: int, seed: int, lo: float, span: float) -> np.ndarray:
 # Which prefill kernel a batch takes, restated from the dispatch rules for
 # choosing test cases (the library answers the same question through
 # slm_attn_prefill_kernel; tests/test_abi.py checks the two agree).
+def split_form(dim, heads, kv_heads, start, n, cus=256):
+    """Which form of the split-bf16 kernel a prefill takes, or None.  With cols
+    (head, 16-row block) columns: hd 128 from 128 keys on, but for the batches
+    of paired_one_head, with key splits up to four columns per CU and paired
+    blocks up to eight; hd 64 from three columns per CU, with key splits up to
+    eight and paired blocks up to sixteen."""
+    hd = dim // heads
+    cols = -(-n // 16) * heads
+    if hd == 128:
+        if start + n < 128 or paired_one_head(dim, heads, kv_heads, n, cus):
+            return None
+        keys, paired = 4, 8
+    elif hd == 64:
+        if cols < 3 * cus:
+            return None
+        keys, paired = 8, 16
+    else:
+        return None
+    return ("split_keys" if cols <= keys * cus else
+            "split_paired" if cols <= paired * cus else "split_consecutive")
+
+
 def takes_key_splits(dim, heads, kv_heads, start, n, cus=256):
     """Whether a prefill takes the one-head key-split kernel (prefill_plan.h):
-    head_dim <= 64, fewer than two workgroups per CU in the
-    head-group tiling, at least 8 key tiles in the heaviest block."""
+    head_dim <= 64 and not the split-bf16 kernel, fewer than two workgroups per
+    CU in the head-group tiling, at least 8 key tiles in the heaviest block."""
     hd = dim // heads
     kv_mul = heads // kv_heads
     hw = 4 if kv_mul % 4 == 0 else 3 if kv_mul % 3 == 0 else 2 if kv_mul % 2 == 0 else 1
     qs = {4: 1, 3: 1, 2: 2, 1: 4}[hw]
     wgs = -(-n // (16 * qs)) * (heads // hw)
-    return hd <= 64 and wgs < 2 * cus and (start + n + 31) // 32 >= 8
+    return (hd <= 64 and split_form(dim, heads, kv_heads, start, n, cus) is None
+            and wgs < 2 * cus and (start + n + 31) // 32 >= 8)
 
 
-def paired_blocks(dim, heads, kv_heads, n, cus=256):
-    """Which paired-block kernel an hd-128 prefill of n rows takes (blocks i
-    and n_qb-1-i per workgroup), or None: for at least 256 rows whose
-    head-group tiling gives at most one workgroup per CU, one head and four
-    key splits ("h1k4") while pairs x heads fit the CUs, else two heads and
-    two key splits ("h2k2") for an even kv_mul while pairs x heads/2 fit."""
+def paired_one_head(dim, heads, kv_heads, n, cus=256):
+    """Whether an hd-128 prefill of n rows takes the f32 kernel of one head,
+    paired blocks (i and n_qb-1-i) and four key splits per workgroup: at least
+    256 rows whose head-group tiling gives at most one workgroup per CU, while
+    pairs x heads fit the CUs."""
     hd = dim // heads
     kv_mul = heads // kv_heads
     hw, qs = (4, 1) if kv_mul % 4 == 0 else (3, 1) if kv_mul % 3 == 0 else \
         (2, 2) if kv_mul % 2 == 0 else (1, 4)
     wgs = -(-n // (16 * qs)) * (heads // hw)
     pairs = (-(-n // 16) + 1) // 2
-    if hd != 128 or n < 256 or wgs > cus:
-        return None
-    if pairs * heads <= cus:
-        return "h1k4"
-    if kv_mul % 2 == 0 and pairs * (heads // 2) <= cus:
-        return "h2k2"
-    return None
-
-
-def paired_dma(dim, heads, kv_heads, n, cus=256):
-    """hd-128 prefills of 512 rows or more with kv_mul a multiple of 4 that
-    the short paired kernels leave take the DMA-fed kernel with paired blocks
-    (blocks i and n_qb-1-i, four heads) when the four-head grid has more
-    workgroups than CUs and the paired grid is at most the CU count or a
-    whole multiple of it."""
-    kv_mul = heads // kv_heads
-    wgs = -(-n // 16) * (heads // 4)
-    pwgs = (-(-n // 16) + 1) // 2 * (heads // 4)
-    return (dim // heads == 128 and kv_mul % 4 == 0 and n >= 512
-            and paired_blocks(dim, heads, kv_heads, n, cus) is None
-            and wgs > cus and (pwgs <= cus or pwgs % cus == 0))
+    return hd == 128 and n >= 256 and wgs <= cus and pairs * heads <= cus
 
 
 def paired_register(dim, heads, kv_heads, start, n, cus=256):
     """Prefills of hd 16-96 with kv_mul a multiple of 4 that the one-head
-    key-split kernel leaves take the four-head register kernel with paired
-    blocks when the four-head grid has more workgroups than CUs and the
-    paired grid is at most one or two per CU."""
+    key-split kernel and the split-bf16 one leave take the four-head kernel
+    with paired blocks when the four-head grid has more workgroups than CUs
+    and the paired grid is at most one or two per CU."""
     hd, kv_mul = dim // heads, heads // kv_heads
     wgs = -(-n // 16) * (heads // 4)
     pwgs = (-(-n // 16) + 1) // 2 * (heads // 4)
-    key_splits = hd <= 64 and wgs < 2 * cus and (start + n + 31) // 32 >= 8
-    return (hd <= 96 and kv_mul % 4 == 0 and not key_splits and wgs > cus
-            and (pwgs <= cus or pwgs == 2 * cus))
+    return (hd <= 96 and kv_mul % 4 == 0 and wgs > cus and (pwgs <= cus or pwgs == 2 * cus)
+            and split_form(dim, heads, kv_heads, start, n, cus) is None
+            and not takes_key_splits(dim, heads, kv_heads, start, n, cus))
 
 
 # Prefill kernels (slm_attn_prefill_kernel, static-lm_amd PREFILL_KERNELS) and
@@ -258,9 +260,9 @@ SWEEP_TARGETED = [
     (768, 16, 16, 0, 40, "one_head"),             # hd 48 MHA
     (576, 9, 3, 0, 512, "key_split"),             # the SmolLM2-135M shape, 512 rows
     (3072, 32, 8, 0, 1024, "paired_four_heads"),  # hd 96 GQA 4, 256 paired workgroups
-    (8192, 64, 16, 3, 2100, "dma"),               # hd 128, 1056 workgroups (not a multiple of 256)
-    (4096, 32, 8, 0, 1024, "dma_paired"),         # the Llama-3-8B shape, 256 paired workgroups
-    (4096, 32, 8, 0, 300, "paired_two_heads"),    # the Llama-3-8B shape, 10 pairs
+    (8192, 64, 16, 3, 2100, "split_consecutive"),  # hd 128, 33 columns per CU
+    (4096, 32, 8, 0, 1024, "split_paired"),       # the Llama-3-8B shape, 8 columns per CU
+    (4096, 32, 8, 0, 300, "split_keys"),          # the Llama-3-8B shape, 2.4 columns per CU
     (4096, 32, 8, 0, 256, "paired_one_head"),     # the Llama-3-8B shape, 8 pairs
 ]
 

@@ -6,8 +6,8 @@ import subprocess
 
 import pytest
 
-from slm_testlib import (SWEEP_TARGETED, load_product, paired_blocks, paired_dma,
-                         paired_register, sweep_random_cases, takes_key_splits)
+from slm_testlib import (SWEEP_TARGETED, load_product, paired_one_head, paired_register,
+                         split_form, sweep_random_cases, takes_key_splits)
 
 P = load_product()
 
@@ -187,7 +187,7 @@ def _plan_grid():
                 {m + d for m in (256, 512, 1024, 2048, 4096, 8192) for d in (-17, -1, 0, 1, 15)})
     for hd in (16, 32, 48, 64, 96, 128, 256):
         for kv_mul in (1, 2, 3, 4, 8):
-            for kvh in (1, 2, 4, 8):
+            for kvh in (1, 2, 4, 8, 64):
                 for cus in (256, 32):
                     for start in (0, 7, 1000):
                         for n in ns:
@@ -201,15 +201,14 @@ def test_prefill_plan_picks_only_compiled_kernels(prefill_plan):
     def compiled(hd, kv_mul, k):
         return {"four_heads": kv_mul % 4 == 0, "three_heads": kv_mul % 3 == 0,
                 "two_heads": kv_mul % 2 == 0, "one_head": True, "key_split": hd <= 64,
-                "paired_four_heads": hd <= 96 and kv_mul % 4 == 0,
-                "dma": hd == 128 and kv_mul % 4 == 0, "dma_paired": hd == 128 and kv_mul % 4 == 0,
-                "paired_two_heads": hd == 128 and kv_mul % 2 == 0,
-                "paired_one_head": hd == 128}[k]
+                "paired_four_heads": hd in (16, 32, 48, 96) and kv_mul % 4 == 0,
+                "paired_one_head": hd == 128, "split_keys": hd in (64, 128),
+                "split_paired": hd in (64, 128), "split_consecutive": hd in (64, 128)}[k]
     grid = list(_plan_grid())
     got = prefill_plan(grid)
     bad = [(c, k) for c, k in zip(grid, got) if not compiled(c[0], c[2], k)]
     assert not bad, bad[:5]
-    assert set(got) == set(P.PREFILL_KERNELS)
+    assert set(got) == set(P.PREFILL_KERNELS.values())
 
 
 def test_prefill_plan_agrees_with_the_restated_rules(prefill_plan):
@@ -221,10 +220,9 @@ def test_prefill_plan_agrees_with_the_restated_rules(prefill_plan):
         dim, kvh = heads * hd, heads // kv_mul
         case = (hd, heads, kv_mul, cus, start, n, k)
         assert (k == "key_split") == takes_key_splits(dim, heads, kvh, start, n, cus), case
-        pb = paired_blocks(dim, heads, kvh, n, cus)
-        assert (k == "paired_one_head") == (pb == "h1k4"), case
-        assert (k == "paired_two_heads") == (pb == "h2k2"), case
-        assert (k == "dma_paired") == paired_dma(dim, heads, kvh, n, cus), case
+        assert (k == "paired_one_head") == paired_one_head(dim, heads, kvh, n, cus), case
+        assert (k if k.startswith("split_") else None) == \
+            split_form(dim, heads, kvh, start, n, cus), case
         assert (k == "paired_four_heads") == paired_register(dim, heads, kvh, start, n, cus), case
 
 
@@ -235,7 +233,7 @@ def test_dispatch_sweep_reaches_every_prefill_kernel(prefill_plan):
              for dim, heads, kvh, start, n, _ in SWEEP_TARGETED]
     got = prefill_plan(cases)
     assert got == [c[5] for c in SWEEP_TARGETED]
-    assert set(got) == set(P.PREFILL_KERNELS)
+    assert set(got) == set(P.PREFILL_KERNELS.values())
     rnd = sweep_random_cases()
     kinds = prefill_plan([(dim // heads, heads, heads // kvh, 256, start, n)
                           for dim, heads, kvh, start, n in rnd])
@@ -251,7 +249,8 @@ def test_prefill_kernel_query_checks_its_arguments():
 
 def test_header_numbers_the_prefill_kernels_like_the_binding():
     text = P.HEADER_PATH.read_text()
-    for i, name in enumerate(P.PREFILL_KERNELS):
+    assert text.count(" SLM_PF_") == len(P.PREFILL_KERNELS)
+    for i, name in P.PREFILL_KERNELS.items():
         assert f"SLM_PF_{name.upper()} = {i}," in text or f"SLM_PF_{name.upper()} = {i} " in text, name
 
 

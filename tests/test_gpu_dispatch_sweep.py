@@ -90,7 +90,7 @@ def test_prefill_kernel_query_rejects_batches_the_prefill_rejects():
     # the same checks and codes as slm_attn_prefill (SLM_ERR_BATCH); a batch
     # ending at max_seq_len is accepted
     with P.AttentionContext(4096, 32, 8, 300, 1, 5e5) as ctx:
-        assert ctx.prefill_kernel(0, 300) == "paired_two_heads"
+        assert ctx.prefill_kernel(0, 300) == "split_keys"
         for start, n in ((0, 0), (-1, 4), (290, 11), (300, 1)):
             with pytest.raises(P.SlmAttnError) as e:
                 ctx.prefill_kernel(start, n)

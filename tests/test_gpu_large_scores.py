@@ -308,14 +308,14 @@ def test_decode_large_scores_closed_form(name, p):
 
 # ---- prefill -----------------------------------------------------------------
 
-# (shape, start, n): the 4096-row Llama-3-8B-shape prefill takes the DMA-fed
-# kernel on 256 CUs; the others the register-prefetch kernel: four heads per
-# workgroup at hd 128, 256 and 32, one head and four query blocks for the hd
-# 128 and hd 96 MHA shapes; the hd 64 (three heads), hd 48 and hd 16 shapes
-# give under two workgroups per CU at these lengths and take the one-head
-# kernel with the key tiles split over four waves; 480 Llama-3-8B-shape rows
-# take the paired-block kernel (two heads, blocks i and n-1-i, two key
-# splits), 256 rows of hd 128 MHA its one-head form (four key splits)
+# (shape, start, n): the Llama-3-8B shape takes the split-bf16 kernel on 256
+# CUs, with consecutive blocks at 4096 rows, paired ones at 1000 and key splits
+# at 480; hd 128 MHA its consecutive form at 2048 rows and the f32 kernel of one
+# head, paired blocks and four key splits at 256.  The others run on f32: four
+# heads per workgroup at hd 256 and (paired) 32, one head and four query blocks
+# for hd 96 MHA; hd 48 and hd 16 give under two workgroups per CU at these
+# lengths and take the one-head kernel with the key tiles split over four
+# waves; 2048 rows of hd 64 in nine heads the split-bf16 one with key splits
 PREFILL_CASES = [("llama3-8b", 0, 4096), ("llama3-8b", 24, 1000), ("llama3-8b", 100, 480),
                  ("hd128-mha", 40, 256), ("smollm2", 0, 2048),
                  ("stories15m", 0, 512), ("hd128-mha", 0, 2048), ("hd256-gqa4", 24, 1000),

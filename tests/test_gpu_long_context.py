@@ -181,21 +181,20 @@ def test_prefill_uniform_scores_every_row(start, n):
 
 
 @pytest.mark.parametrize("dim,heads,kv_heads,start,n", [
-    (4096, 32, 8, 7, 4111),   # 129 query blocks of 32: the last holds 15 rows, so its
-                              # second 16-row wave has none but joins every DMA and barrier
+    (4096, 32, 8, 7, 4111),   # 129 pairs of query blocks: the last holds 15 rows, so its
+                              # second block's waves have none but join every tile and barrier
     (8192, 64, 8, 0, 2100),   # kv_mul 8: two workgroups' head groups share each KV head
 ])
-def test_dma_prefill_unaligned_every_row(dim, heads, kv_heads, start, n):
-    """Zero keys through the DMA-fed prefill kernel (hd 128, four query heads
-    per workgroup, at least four workgroups per CU on 256 CUs) at row counts
-    that are not multiples of its 32-row query block: every row against the
-    closed form."""
+def test_split_prefill_unaligned_every_row(dim, heads, kv_heads, start, n):
+    """Zero keys through the split-bf16 prefill kernel with consecutive blocks
+    (hd 128, four query heads and two blocks per workgroup) at row counts that
+    are not multiples of its 32 rows: every row against the closed form."""
     hd = dim // heads
     kv_dim = hd * kv_heads
     total = start + n
     v_all = v_int_rows(0, total, kv_dim)
     cums = np.cumsum(v_all, axis=0)
-    log(f"DMA prefill {heads}/{kv_heads} heads, rows {start}..{total - 1}")
+    log(f"split prefill {heads}/{kv_heads} heads, rows {start}..{total - 1}")
     with P.AttentionContext(dim, heads, kv_heads, total, 1, 5e5) as ctx:
         q = torch.from_numpy(gen([23, start], (total, dim))).cuda()
         k = torch.zeros(total, kv_dim, device="cuda")
@@ -212,15 +211,15 @@ def test_dma_prefill_unaligned_every_row(dim, heads, kv_heads, start, n):
     want = (cums[rows].reshape(n, kv_heads, hd).astype(np.float64)
             / (rows + 1)[:, None, None].astype(np.float64))
     want = np.repeat(want, heads // kv_heads, axis=1).reshape(n, dim)
-    check(got, want, f"DMA prefill rows {start}..{total - 1}")
+    check(got, want, f"split prefill rows {start}..{total - 1}")
 
 def test_prefill_and_decode_past_row_2_pow_20():
     """One layer's K slice past 4 GiB (1,048,600 rows of kv_dim 1024, an
     8.6 GB cache): zero keys and V integers 0..15 (every sum below 2^24
-    stays exact).  The 32-row prefill takes the register-prefetch kernel,
-    the 4096-row one the DMA kernel; both end at row 1,048,599, so their
-    first tiles' buffer ranges would have wrapped in 32 bits (to 8 and 24
-    rows), reading the other rows of those tiles as zeros.  Every row of
+    stays exact).  The 32-row prefill takes the split-bf16 kernel with key
+    splits, the 4096-row one its consecutive form; both end at row 1,048,599,
+    so their first tiles' buffer ranges would have wrapped in 32 bits (to 8
+    and 24 rows), reading the other rows of those tiles as zeros.  Every row of
     both against the closed form, then one decode at the last position."""
     msl = (1 << 20) + 24
     mod = 16

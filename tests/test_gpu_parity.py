@@ -17,8 +17,8 @@ import pytest
 
 from oracle import py_oracle as orc
 from slm_testlib import (WORKLOADS, Workload, assert_bitwise, assert_close, gen, layer_inputs,
-                         load_product, paired_blocks, paired_dma, paired_register,
-                         prefilled_rows, takes_key_splits)
+                         load_product, paired_one_head, paired_register, prefilled_rows,
+                         split_form, takes_key_splits)
 
 P = load_product()
 pytestmark = pytest.mark.gpu
@@ -114,8 +114,8 @@ def test_llama3_shape_prefill4096_then_decode():
 
 def test_llama3_shape_prefill4096_continued_at_300():
     # A 4096-row prefill continued at start 300: on 256 CUs this size and
-    # shape take the prefill kernel that stages K/V tiles by DMA, whose key
-    # range then starts past the first tile boundary.  K/V rows bit for bit,
+    # shape take the split-bf16 kernel with consecutive blocks, whose rows
+    # then start past the first tile boundary.  K/V rows bit for bit,
     # sampled rows against the oracle over the same cache.
     w = WORKLOADS["c4"]
     cfg = w.cfg()
@@ -139,20 +139,22 @@ def test_llama3_shape_prefill4096_continued_at_300():
 
 @pytest.mark.parametrize("dim,heads,kv_heads,start,n", [(4096, 32, 8, 7, 4111),
                                                         (8192, 64, 8, 0, 2100)])
-def test_dma_prefill_unaligned_against_oracle(dim, heads, kv_heads, start, n):
-    # The DMA-staged prefill kernel at row counts that leave a partial last
-    # 32-row query block (4111 rows: 15 in the last block, whose second wave
-    # has none) and with two head groups per KV head (kv_mul 8).  K/V rows bit
+def test_split_prefill_unaligned_against_oracle(dim, heads, kv_heads, start, n):
+    # The split-bf16 kernel with consecutive blocks at row counts that leave a
+    # partial last pair of blocks (4111 rows: 15 in the last block, whose
+    # partner has none) and with two head groups per KV head (kv_mul 8).  K/V rows bit
     # for bit; rows around the block edges and the last rows against the
     # oracle over the same cache.
-    w = Workload("dma-unaligned", dim, heads, kv_heads, start + n, 1, 5e5, n, 0)
+    assert split_form(dim, heads, kv_heads, start, n) == "split_consecutive"
+    w = Workload("unaligned", dim, heads, kv_heads, start + n, 1, 5e5, n, 0)
     cfg = w.cfg()
     rows = start + n
     q = gen([94, dim], (rows, dim))
     k = gen([95, dim], (rows, w.kv_dim))
     v = gen([96, dim], (rows, w.kv_dim))
     with make_ctx(w) as ctx:
-        log(f"DMA prefill {heads}/{kv_heads} heads: {n} rows at start {start}")
+        assert ctx.prefill_kernel(start, n) == "split_consecutive"
+        log(f"split prefill {heads}/{kv_heads} heads: {n} rows at start {start}")
         if start:
             ctx.prefill(0, 0, q[:start], k[:start], v[:start])
         g = ctx.prefill(0, start, q[start:], k[start:], v[start:])
@@ -163,14 +165,14 @@ def test_dma_prefill_unaligned_against_oracle(dim, heads, kv_heads, start, n):
         for b in (0, 1, 15, 16, 31, 32, 33, 1000, n - 33, n - 21, n - 20, n - 17, n - 16,
                   n - 15, n - 2, n - 1):
             p = start + b
-            assert_close(g[b], om.attend(0, q[p], p), what=f"DMA prefill row {p}")
+            assert_close(g[b], om.attend(0, q[p], p), what=f"split prefill row {p}")
 
 
 @pytest.mark.parametrize("start,n", [(0, 512), (0, 1000), (333, 700), (3000, 64), (40, 30),
                                      (31, 2)])
 def test_llama3_shape_short_prefill_every_row(start, n):
-    # Llama-3-8B-shape prefills below the size that takes the DMA-staged
-    # kernel (the register-prefetch kernel, 16-row blocks of four heads),
+    # Llama-3-8B-shape prefills of up to 1000 rows (the split-bf16 kernel with
+    # key splits or paired blocks; below row 128 the f32 kernel of four heads),
     # from the start of the cache and continued past it at tile-unaligned
     # starts (a block's first rows then share their diagonal tile with the
     # previous call's rows).  Every row against the oracle, K/V rows bit for
@@ -194,20 +196,27 @@ def test_llama3_shape_short_prefill_every_row(start, n):
         assert_close(g, ref, what=f"prefill of {n} rows at {start}")
 
 
-@pytest.mark.parametrize("dim,heads,kv_heads,start,n,variant", [
-    (4096, 32, 8, 0, 256, "h1k4"),     # 16 blocks: 8 pairs of one head
-    (4096, 32, 32, 17, 256, "h1k4"),   # MHA (the Llama-2-7B layout), unaligned start
-    (2048, 16, 16, 0, 300, "h1k4"),    # MHA, 19 blocks: the middle pair's second block is its first
-    (1024, 8, 4, 0, 700, "h1k4"),      # kv_mul 2, 44 blocks
-    (4096, 32, 8, 0, 300, "h2k2"),     # 19 blocks, two heads
-    (4096, 32, 8, 37, 471, "h2k2"),    # unaligned start and a partial last block
-    (4096, 32, 8, 1000, 512, "h2k2"),  # a long prefix: every block's keys span 48 tiles
-    (2048, 16, 2, 0, 777, "h2k2"),     # kv_mul 8: two head pairs per KV head, 49 blocks
-    (1024, 8, 4, 13, 1500, "h2k2"),    # kv_mul 2
+@pytest.mark.parametrize("dim,heads,kv_heads,start,n,kernel", [
+    (4096, 32, 8, 0, 256, "paired_one_head"),     # 16 blocks: 8 pairs of one head
+    (4096, 32, 32, 17, 256, "paired_one_head"),   # MHA (the Llama-2-7B layout), unaligned start
+    (2048, 16, 16, 0, 300, "paired_one_head"),    # MHA, 19 blocks: the middle pair's second block is its first
+    (1024, 8, 4, 0, 700, "paired_one_head"),      # kv_mul 2, 44 blocks
+    (4096, 32, 8, 0, 300, "split_keys"),     # 19 blocks
+    (4096, 32, 8, 37, 471, "split_keys"),    # unaligned start and a partial last block
+    (4096, 32, 8, 1000, 512, "split_keys"),  # a long prefix: every block's keys span 48 tiles
+    (2048, 16, 2, 0, 777, "split_keys"),     # kv_mul 8: four head pairs per KV head, 49 blocks
+    (1024, 8, 4, 13, 1500, "split_keys"),    # kv_mul 2
+    (4096, 32, 8, 5, 1020, "split_paired"),  # 64 blocks, 8 columns per CU, a partial last block
+    (2048, 16, 4, 0, 1520, "split_paired"),  # 95 blocks: the middle pair's second block is its first
+    (2048, 16, 2, 19, 1100, "split_paired"),  # kv_mul 8
+    (4096, 32, 8, 5, 2040, "split_consecutive"),  # 128 blocks, a partial last block
+    (2048, 32, 8, 0, 400, "split_keys"),     # hd 64 (the Llama-3.2-1B layout), 25 blocks
+    (2048, 32, 8, 0, 2048, "split_paired"),  # hd 64, 16 columns per CU
 ])
-def test_prefill_paired_blocks_every_row(dim, heads, kv_heads, start, n, variant):
+def test_prefill_paired_and_split_every_row(dim, heads, kv_heads, start, n, kernel):
     # every row against the oracle, K/V rows bit for bit
-    assert paired_blocks(dim, heads, kv_heads, n) == variant
+    assert (paired_one_head(dim, heads, kv_heads, n) if kernel == "paired_one_head"
+            else split_form(dim, heads, kv_heads, start, n) == kernel)
     rows = start + n
     cfg = orc.Cfg(dim, heads, kv_heads, rows, 1, 5e5)
     q = gen([102, start, n], (rows, dim))
@@ -215,36 +224,8 @@ def test_prefill_paired_blocks_every_row(dim, heads, kv_heads, start, n, variant
     v = gen([104, start, n], (rows, cfg.kv_dim))
     om = orc.OracleModel(cfg)
     with P.AttentionContext(dim, heads, kv_heads, rows, 1, 5e5) as ctx:
-        log(f"paired-block prefill {heads}/{kv_heads} heads: {n} rows at start {start}")
-        assert ctx.prefill_kernel(start, n) == {"h1k4": "paired_one_head",
-                                                "h2k2": "paired_two_heads"}[variant]
-        if start:
-            ctx.prefill(0, 0, q[:start], k[:start], v[:start])
-            om.append(0, 0, k[:start], v[:start])
-        g = ctx.prefill(0, start, q[start:], k[start:], v[start:])
-        ref = om.prefill(0, start, q[start:], k[start:], v[start:])
-        assert_bitwise(ctx.kv_read(0, 0, 0, rows), om.k_cache(0)[:rows], "K rows")
-        assert_bitwise(ctx.kv_read(0, 1, 0, rows), om.v_cache(0)[:rows], "V rows")
-        assert_close(g, ref, what=f"prefill of {n} rows at {start}")
-
-
-@pytest.mark.parametrize("dim,heads,kv_heads,start,n", [
-    (4096, 32, 8, 5, 2040),    # 128 blocks, 512 workgroups (two per CU), a partial last block
-    (2048, 16, 4, 0, 1520),    # 95 blocks: the middle pair's second block is its first
-    (2048, 16, 2, 19, 1100),   # kv_mul 8: two workgroups' heads share each KV head
-])
-def test_prefill_paired_dma_every_row(dim, heads, kv_heads, start, n):
-    # every row against the oracle, K/V rows bit for bit
-    assert paired_dma(dim, heads, kv_heads, n)
-    rows = start + n
-    cfg = orc.Cfg(dim, heads, kv_heads, rows, 1, 5e5)
-    q = gen([105, start, n], (rows, dim))
-    k = gen([106, start, n], (rows, cfg.kv_dim))
-    v = gen([107, start, n], (rows, cfg.kv_dim))
-    om = orc.OracleModel(cfg)
-    with P.AttentionContext(dim, heads, kv_heads, rows, 1, 5e5) as ctx:
-        log(f"paired-block DMA prefill {heads}/{kv_heads} heads: {n} rows at start {start}")
-        assert ctx.prefill_kernel(start, n) == "dma_paired"
+        log(f"{kernel} prefill hd {dim // heads} {heads}/{kv_heads} heads: {n} rows at start {start}")
+        assert ctx.prefill_kernel(start, n) == kernel
         if start:
             ctx.prefill(0, 0, q[:start], k[:start], v[:start])
             om.append(0, 0, k[:start], v[:start])
@@ -258,7 +239,7 @@ def test_prefill_paired_dma_every_row(dim, heads, kv_heads, start, n):
 @pytest.mark.parametrize("dim,heads,kv_heads,start,n", [
     (3072, 32, 8, 0, 1000),   # hd 96: 63 blocks, the middle pair's second block is its first
     (3072, 32, 8, 9, 2040),   # hd 96: 128 blocks, two workgroups per CU, partial last block
-    (2048, 32, 8, 0, 2048),   # hd 64 (the Llama-3.2-1B layout)
+    (1536, 32, 8, 0, 2048),   # hd 48
     (1024, 32, 8, 3, 1015),   # hd 32: 64 blocks, the last partial
     (512, 32, 8, 0, 2048),    # hd 16
 ])
@@ -272,7 +253,7 @@ def test_prefill_paired_register_every_row(dim, heads, kv_heads, start, n):
     v = gen([110, start, n], (rows, cfg.kv_dim))
     om = orc.OracleModel(cfg)
     with P.AttentionContext(dim, heads, kv_heads, rows, 1, 5e5) as ctx:
-        log(f"paired-block register prefill hd {dim // heads}: {n} rows at start {start}")
+        log(f"paired-block prefill hd {dim // heads}: {n} rows at start {start}")
         assert ctx.prefill_kernel(start, n) == "paired_four_heads"
         if start:
             ctx.prefill(0, 0, q[:start], k[:start], v[:start])

@@ -4,22 +4,25 @@ cannot be split."""
 import numpy as np
 import pytest
 
-from slm_testlib import gen, load_product
+from slm_testlib import gen, load_product, split_form
 
 P = load_product()
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
 
-def run(heads, kvh, start, q, k, v):
-    """attend_batch of rotated q [n][dim] over cache rows 0..start+n-1."""
+def run(heads, kvh, start, q, k, v, form=None):
+    """attend_batch of rotated q [n][dim] over cache rows 0..start+n-1, in the
+    form that the dispatch rules give the split kernel."""
     rows, n = k.shape[0], q.shape[0]
+    form = form or split_form(q.shape[1], heads, kvh, start, n)
     with P.AttentionContext(q.shape[1], heads, kvh, max(rows, 16), 1) as ctx:
         ctx.kv_write(0, 0, 0, k)
         ctx.kv_write(0, 1, 0, v)
         qd = torch.from_numpy(q).cuda()
         out = torch.full_like(qd, float("nan"))
         torch.cuda.synchronize()
+        assert ctx.prefill_kernel(start, n) == form
         ctx.attend_batch_dev(0, start, n, qd.data_ptr(), out.data_ptr())
         ctx.sync()
         return out.cpu().numpy()
@@ -43,28 +46,36 @@ def attend64(heads, kvh, start, q, k, v):
     return out, mag, smax
 
 
-# hd, heads, kv_heads, start, n: one, two, three, four and eight heads per KV head;
-# key splits, paired and consecutive blocks; block and tile edges (15/16/17
-# rows, 127 to 129 and 159 to 161 keys), odd and even block counts
-CASES = [
-    (128, 2, 1, 112, 16), (128, 2, 1, 111, 17), (128, 2, 1, 113, 15), (128, 4, 1, 0, 128),
-    (128, 4, 1, 0, 129), (128, 1, 1, 100, 28), (128, 1, 1, 127, 33), (128, 3, 1, 0, 160),
-    (128, 3, 3, 30, 131), (128, 8, 1, 96, 65), (128, 12, 4, 0, 250), (128, 2, 2, 1000, 2),
-    (128, 4, 2, 500, 47), (128, 32, 8, 0, 545), (128, 32, 32, 3, 528), (128, 32, 8, 0, 1025),
-    (128, 24, 8, 40, 1400), (128, 32, 16, 0, 1040),
-    (64, 32, 8, 0, 380), (64, 32, 8, 0, 384), (64, 24, 8, 5, 511), (64, 32, 8, 1, 1023),
-    (64, 32, 32, 0, 1040), (64, 36, 12, 0, 1100), (64, 32, 8, 0, 2065), (64, 48, 6, 3, 1403),
-]
+# hd, heads, kv_heads, start, n: every form with one, two and (consecutive) four
+# heads per workgroup, of one, two, three, four, eight and more heads per KV
+# head; block and tile edges (15/16/17 rows, 127 to 129 and 159 to 161 keys),
+# odd and even block counts
+CASES = {
+    "split_keys": [
+        (128, 2, 1, 112, 16), (128, 2, 1, 111, 17), (128, 2, 1, 113, 15), (128, 4, 1, 0, 128),
+        (128, 4, 1, 0, 129), (128, 1, 1, 100, 28), (128, 1, 1, 127, 33), (128, 3, 1, 0, 160),
+        (128, 3, 3, 30, 131), (128, 8, 1, 96, 65), (128, 12, 4, 0, 250), (128, 2, 2, 1000, 2),
+        (128, 4, 2, 500, 47), (64, 32, 8, 0, 380), (64, 32, 8, 0, 384), (64, 24, 8, 5, 511),
+        (64, 32, 8, 1, 1023)],
+    "split_paired": [
+        (128, 32, 8, 0, 545), (128, 32, 32, 3, 528), (64, 32, 32, 0, 1040),
+        (64, 36, 12, 0, 1100), (64, 32, 16, 0, 1300)],
+    "split_consecutive": [
+        (128, 32, 8, 0, 1025), (128, 24, 8, 40, 1400), (128, 32, 16, 0, 1040),
+        (64, 32, 8, 0, 2065), (64, 48, 6, 3, 1403), (64, 32, 32, 0, 2065),
+        (64, 33, 11, 0, 2030), (64, 32, 16, 1, 2080)],
+}
+CASES = [(*c, form) for form, cases in CASES.items() for c in cases]
 
 
-@pytest.mark.parametrize("hd,heads,kvh,start,n", CASES)
-def test_against_float64(hd, heads, kvh, start, n):
+@pytest.mark.parametrize("hd,heads,kvh,start,n,form", CASES)
+def test_against_float64(hd, heads, kvh, start, n, form):
     rows = start + n
     q = gen([71, heads, start, n], (n, heads * hd)) * np.float32(4)
     k = gen([72, heads, start, n], (rows, kvh * hd)) * np.float32(2)
     v = gen([73, heads, start, n], (rows, kvh * hd))
     ref, mag, smax = attend64(heads, kvh, start, q, k, v)
-    got = run(heads, kvh, start, q, k, v)
+    got = run(heads, kvh, start, q, k, v, form)
     # Roundings of 2^-24: six per 32-key tile in an output sum and one in the
     # row sum, per score 24 accumulations (of partial sums taken as at most
     # twice the largest score, in log2 units) and the pre-scaled q, and a few
@@ -82,7 +93,7 @@ def test_against_float64(hd, heads, kvh, start, n):
 def test_many_heads_before_row_128(start, n):
     """Batches too short for the split kernel with so many heads that they fill
     the CUs several times over."""
-    test_against_float64(128, 1024, 64, start, n)
+    test_against_float64(128, 1024, 64, start, n, "four_heads")
 
 
 @pytest.mark.parametrize("hd,heads,kvh,start,n", [(128, 2, 1, 100, 60), (128, 32, 8, 0, 600),
