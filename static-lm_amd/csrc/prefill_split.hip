@@ -40,10 +40,10 @@
 // bf16's exponents.  The splitting therefore keeps the largest magnitudes of q,
 // K and V, and a wave computes its rows again in f32 from the cache
 // (attend_f32, attend_plain) if a result is not finite, q or K reach 2^64, or
-// an output sum is so small beside V's values that bits lost in P or V could
-// show (least_sum).  Looking costs 1-2% (Llama-3-8B shape, per call: 4096 rows
-// 680 -> 689 us, 777 rows at start 1000 96.7 -> 98.7), computing again several
-// times the call.
+// the terms of an output sum are so small beside V's values that bits lost in P
+// or V could show (least_sum).  Looking costs 1-2% (Llama-3-8B shape, per call:
+// 4096 rows 677 -> 682 us, 777 rows at start 1000 96.1 -> 97.7), computing again
+// several times the call.
 #include <math.h>
 
 #include "attn_common.h"
@@ -516,6 +516,7 @@ __global__ __launch_bounds__(64 * QS * HW * KSP, HD == 64 ? 4 : 2) void prefill_
             mk[k] = s_merge[((k - 1) * NWS + ws) * NR * 64 + lane + 64 * (NR - 2)];
             mx = fmaxf(mx, mk[k]);
         }
+        om = mx;  // the sums' common offset
         const float s0 = __builtin_amdgcn_exp2f(m - mx);
         l *= s0;
 #pragma unroll
@@ -533,17 +534,61 @@ __global__ __launch_bounds__(64 * QS * HW * KSP, HD == 64 ? 4 : 2) void prefill_
     }
 
     if (wave_rows == 0) return;
+    // normalise and store: lane holds out[row][16 dt + 4 lg + (0..3)]
+    auto store = [&]() __attribute__((always_inline)) {
+        const float inv = 1.0f / rows_sum(l);
+        if (!row_ok) return;
+        float* dst = p.out + (long)row * p.dim + head * HD + 4 * lg;
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt)
+            *reinterpret_cast<float4*>(dst + 16 * dt) =
+                make_float4(o[dt][0] * inv, o[dt][1] * inv, o[dt][2] * inv, o[dt][3] * inv);
+    };
+    store();
+
+    // Whether the planes held enough of the operands (bf16's exponents end at
+    // 2^-126, and planes below that may count as zero): with kv_len keys,
+    // probabilities up to 2^kLazyRescale and values up to top, an output sum is
+    // off by less than kv_len * (top + 2^kLazyRescale) * 2^-122, which is below
+    // the roundings of a sum whose terms' magnitudes add up to least_sum(top);
+    // a score of operands below 2^64 by less than 2^-50.
+    auto least_sum = [&](float top) {
+        return (float)kv_len * fmaf(top, 0x1p-96f, 0x1p-96f * (1 << (int)kLazyRescale));
+    };
+    float z = l * 0.0f;  // NaN once any of the row's values is not finite
+    float least = INFINITY;
+#pragma unroll
+    for (int i = 0; i < NDT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            z = fmaf(o[i][r], 0.0f, z);
+            least = fminf(least, fabsf(o[i][r]));
+        }
+    top_k = top_v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        top_k = maximum(top_k, sm.raw[w * kWaveRaw + 64]);
+        top_v = maximum(top_v, sm.raw[w * kWaveRaw + 65]);
+    }
+    bool again = row_ok && (z != z || !(top_k < 0x1p64f));
+    const bool low = row_ok && !(least >= least_sum(top_v));
+    if (!__any(again || low)) return;
+
+    int g8 = lg;
+    asm volatile("" : "+v"(g8));  // made here, not held through the loop above: registers
+    g8 *= 8;
     // A tile in f32 from the cache rows, on f32 matrix instructions where every
     // query of the wave sees all its keys (step j of a product takes one dim or
     // key from each lane group) ...
-    auto attend_f32 = [&](int kb, const float (&x)[NKS][8]) __attribute__((always_inline)) {
+    auto attend_f32 = [&](int kb, const float (&x)[NKS][8], bool abs_v)
+                          __attribute__((always_inline)) {
         v4f s[2] = {negm, negm};
-        const float* kr = kg + (long)(kb + lr) * p.kv_dim + 8 * lg;
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
             for (int kk = 0; kk < 2; ++kk) {
-                const float* src = kr + (long)(16 * kk) * p.kv_dim + 32 * ks;
+                const long r = min(kb + 16 * kk + lr, kv_len - 1);
+                const float* src = kg + r * p.kv_dim + 32 * ks + g8;
                 const float4 a = ld4(src), b = ld4(src + 4);
                 const float y[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
@@ -551,14 +596,17 @@ __global__ __launch_bounds__(64 * QS * HW * KSP, HD == 64 ? 4 : 2) void prefill_
                     s[kk] = __builtin_amdgcn_mfma_f32_16x16x4f32(y[i], x[ks][i], s[kk], 0, 0, 0);
             }
         softmax(kb, s);
-        const float* vr = vg + (long)(kb + 4 * lg) * p.kv_dim + lr;
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
+        for (int j = 0; j < 8; ++j) {
+            const long r = min(kb + 4 * lg + 16 * (j >> 2) + (j & 3), kv_len - 1);
+            const float* src = vg + r * p.kv_dim + lr;
 #pragma unroll
-            for (int dt = 0; dt < NDT; ++dt)
-                o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                    vr[(long)(16 * (j >> 2) + (j & 3)) * p.kv_dim + 16 * dt],
-                    s[j >> 2][j & 3], o[dt], 0, 0, 0);
+            for (int dt = 0; dt < NDT; ++dt) {
+                const float v = src[16 * dt];
+                o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(abs_v ? fabsf(v) : v,
+                                                            s[j >> 2][j & 3], o[dt], 0, 0, 0);
+            }
+        }
     };
     // ... and a key at a time on the diagonal: masked keys take no part in the sums.
     auto attend_plain = [&](int kb, const float (&x)[NKS][8]) __attribute__((always_inline)) {
@@ -567,7 +615,7 @@ __global__ __launch_bounds__(64 * QS * HW * KSP, HD == 64 ? 4 : 2) void prefill_
         for (int kk = 0; kk < 2; ++kk) s[kk] = v4f{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
 #pragma unroll 1
         for (int k = 0; k < KT && kb + k < kv_len; ++k) {
-            const float* kr = kg + (long)(kb + k) * p.kv_dim + 8 * lg;
+            const float* kr = kg + (long)(kb + k) * p.kv_dim + g8;
             float d = 0.0f;
 #pragma unroll
             for (int ks = 0; ks < NKS; ++ks) {
@@ -602,72 +650,52 @@ __global__ __launch_bounds__(64 * QS * HW * KSP, HD == 64 ? 4 : 2) void prefill_
             }
         }
     };
-    // Where the planes may not hold enough of an operand (bf16's exponents end
-    // at 2^-126, and planes below that may count as zero): with kv_len keys,
-    // probabilities up to 2^kLazyRescale and values up to top, an output sum is
-    // off by less than kv_len * (top + 2^kLazyRescale) * 2^-122, which is in
-    // f32's last bits of a sum of at least least_sum(top); a score of operands
-    // below 2^64 by less than 2^-50.
-    float lt = rows_sum(l);
-    auto least_sum = [&](float top) {
-        return (float)kv_len * fmaf(top, 0x1p-96f, 0x1p-96f * (1 << (int)kLazyRescale));
-    };
-    float z = lt * 0.0f;  // NaN once any of the row's values is not finite
-    float least = INFINITY;
+    float x[NKS][8];
 #pragma unroll
-    for (int i = 0; i < NDT; ++i)
+    for (int ks = 0; ks < NKS; ++ks) load_q8(ks, x[ks]);
+    if (!__any(again)) {
+        // Small sums are mostly zeros of dims without values, or sums that
+        // cancelled out (one in 10^7 does, to exactly zero).  The first tile's
+        // terms usually reach least_sum.
+        uint32_t small = 0;  // which of this lane's sums
+        auto by_dim = [&](auto at_each) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            z = fmaf(o[i][r], 0.0f, z);
-            least = fminf(least, fabsf(o[i][r]));
-        }
-    top_k = top_v = 0.0f;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-        top_k = maximum(top_k, sm.raw[w * kWaveRaw + 64]);
-        top_v = maximum(top_v, sm.raw[w * kWaveRaw + 65]);
-    }
-    bool again = z != z || !(top_k < 0x1p64f);
-    if (!again && !(least >= least_sum(top_v))) {
-        // by dim: a dim whose values are all zero has a sum of zero
-#pragma unroll
-        for (int i = 0; i < NDT; ++i) {
-            const int d = 16 * i + 4 * lg;
-            float t[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            for (int i = 0; i < NDT; ++i) {
+                float t[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // largest value of dims 16 i + 4 lg + ..
 #pragma unroll 1
-            for (int j = 0; j < NT / HD; ++j) {
-                const int at = j * HD + d;
-                const float4 x = ld4(&sm.raw[(at >> 6) * kWaveRaw + (at & 63)]);
-                t[0] = maximum(t[0], x.x), t[1] = maximum(t[1], x.y);
-                t[2] = maximum(t[2], x.z), t[3] = maximum(t[3], x.w);
+                for (int j = 0; j < NT / HD; ++j) {
+                    const int at = j * HD + 16 * i + 4 * lg;
+                    const float4 y = ld4(&sm.raw[(at >> 6) * kWaveRaw + (at & 63)]);
+                    t[0] = maximum(t[0], y.x), t[1] = maximum(t[1], y.y);
+                    t[2] = maximum(t[2], y.z), t[3] = maximum(t[3], y.w);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) at_each(i, r, t[r]);
             }
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                again |= t[r] != 0.0f && !(fabsf(o[i][r]) >= least_sum(t[r]));
-        }
-    }
-    if (__any(row_ok && again)) {
+        };
+        by_dim([&](int i, int r, float top) {
+            if (low && top != 0.0f && !(fabsf(o[i][r]) >= least_sum(top))) small |= 1u << (4 * i + r);
+        });
+        if (!__any(small)) return;
+        const float offset = om;
         reset();
-        float x[NKS][8];
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) load_q8(ks, x[ks]);
-        int kb = 0;
-#pragma unroll 1
-        for (; kb + KT - 1 <= p.start + q0; kb += KT) attend_f32(kb, x);
-#pragma unroll 1
-        for (; kb <= wave_last_pos; kb += KT) attend_plain(kb, x);
-        lt = rows_sum(l);
+        om = offset;
+        negm = v4f{-om, -om, -om, -om};
+        lim = INFINITY;  // om stays
+        attend_f32(0, x, true);
+        by_dim([&](int i, int r, float top) {
+            if (small >> (4 * i + r) & 1) again |= !(o[i][r] >= least_sum(top));
+        });
+        if (!__any(again)) return;
     }
 
-    // normalise and store: lane holds out[row][16 dt + 4 lg + (0..3)]
-    if (row_ok) {
-        const float inv = 1.0f / lt;
-        float* dst = p.out + (long)row * p.dim + head * HD + 4 * lg;
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt)
-            *reinterpret_cast<float4*>(dst + 16 * dt) =
-                make_float4(o[dt][0] * inv, o[dt][1] * inv, o[dt][2] * inv, o[dt][3] * inv);
-    }
+    reset();
+    int kb = 0;
+#pragma unroll 1
+    for (; kb + KT - 1 <= p.start + q0; kb += KT) attend_f32(kb, x, false);
+#pragma unroll 1
+    for (; kb <= wave_last_pos; kb += KT) attend_plain(kb, x);
+    store();
 }
 
 template <int HD, int HW, int QS, int KSP, bool PAIR>

@@ -208,3 +208,22 @@ def test_values_below_the_least_bf16(hd, heads, kvh, start, n):
     # as test_small_values
     bound = (2 * rows + 2 * (hd / 4 + 3) * 1.4427 * smax + 16) * 2.0 ** -24
     assert (np.abs(got - ref) <= bound * mag + rows * 2.0 ** -150).all()
+
+
+@pytest.mark.parametrize("tiny", [False, True])
+@pytest.mark.parametrize("hd,heads,kvh,start,n", RANGE_CASES)
+def test_sums_that_cancel(hd, heads, kvh, start, n, tiny):
+    """Equal probabilities of values that cancel in pairs, so that every other
+    row's sums are zero; beside values too small for bf16, in one dim of 16."""
+    rows = start + n
+    q = np.zeros((n, heads * hd), np.float32)
+    k = gen([88, n], (rows, kvh * hd))
+    v = gen([89, n], (rows, kvh * hd))
+    v[1::2] = -v[:rows // 2 * 2:2]
+    if tiny:
+        v[:, 5::16] = np.abs(v[:, 5::16]) * np.float32(2.0 ** -138)
+    ref, mag, _ = attend64(heads, kvh, start, q, k, v)
+    got = run(heads, kvh, start, q, k, v)
+    # Roundings of 2^-24, one per key in the output and row sums; of 2^-150, one per key
+    bound = (2 * rows + 16) * 2.0 ** -24
+    assert (np.abs(got - ref) <= bound * mag + (rows * 2.0 ** -150 if tiny else 0)).all()
