@@ -40,6 +40,37 @@ inline PrefillTiling prefill_tiling(int kv_mul) {
     return {1, 4};
 }
 
+// Whether the split kernel takes a prefill of hd 64 with `cols` (head, 16-row
+// block) columns.  Its arithmetic per key tile is half that of hd 128 behind the
+// same set-up and barriers, so it takes more columns to win, and the f32
+// kernel's four key splits serve what does not fill the CUs: from three columns
+// per CU (32 heads in 8 KV heads: 256 rows, two per CU, 13.8 against 12.5 us in
+// f32, 384 rows 17.6 against 20.8, 512 rows 20.8 against 26.7).  Key splits up
+// to eight columns per CU (16 heads, 2048 rows: 79.7 us, paired 81.4, f32 109.9;
+// 3000 rows: 152, 139, 201), paired blocks up to sixteen (32 heads, 2048 rows:
+// 106 us, consecutive 112, f32 150; 3000 rows: 214, 200, 312).
+//
+// With one workgroup (four columns) per CU its time follows the heaviest
+// block's keys (10.5 us + 23 ns a key), that of the f32 kernel, whose small
+// workgroups fill in behind each other, the keys that all columns see together.
+// So long histories of few columns need more of them, counted by the keys that
+// the average row sees: split against f32, start 0, at 3.0 / 3.5 / 3.9 columns
+// per CU 4 heads 81.8 / 95.1 / 105.6 against 62.4 / 83.5 / 103.3 us (3072 to 3994
+// rows), 6 heads 57.8 / 67.3 / 74.3 against 48.8 / 64.5 / 75.6, 9 heads 42.2 /
+// 48.4 / - against 39.5 / 48.5 / -, 12 heads (1024 rows) 32.9 against 33.0; 8
+// heads, 1536 rows at start 600 63.0 against 65.2.  With a second workgroup on
+// some of the CUs, at 4.1 / 4.5 / 5.0: 8 heads 67.6 / 73.8 / 81.9 against 63.2 /
+// 71.5 / 84.1, 12 heads 49.4 / 54.0 against 49.0 / 54.7, 14 heads (1200 rows) 41.8
+// against 42.8.
+inline bool hd64_splits(long cols, int cus, int start, int n) {
+    if (cols < 3L * cus) return false;
+    const double keys = (double)start + n;
+    const double seen = (double)cols / cus * (start + 0.5 * n) / keys;
+    if (cols <= 4L * cus) return seen >= 2.2 - 768.0 / keys;
+    const double least = 3.0 - 1280.0 / keys;
+    return seen >= (least < 2.5 ? least : 2.5);
+}
+
 // Which kernel a prefill of n rows from row `start` runs, for head_dim,
 // num_heads query heads (kv_mul per KV head) on a device of `cus` CUs: a pure
 // function of the batch, the shape and the CU count.  The launcher and the
@@ -78,16 +109,7 @@ inline PrefillKernel prefill_plan(int head_dim, int num_heads, int kv_mul, int c
                    : cols <= 8L * cus ? PrefillKernel::kSplitPaired
                                       : PrefillKernel::kSplitConsecutive;
     }
-    // Half the arithmetic per key tile of hd 128 behind the same set-up and
-    // barriers, so at hd 64 it takes more columns to win, and the f32 kernel's
-    // four key splits serve what does not fill the CUs: from three columns per
-    // CU (32 heads in 8 KV heads: 256 rows, two per CU, 13.8 against 12.5 us in
-    // f32, 384 rows 17.6 against 20.8, 512 rows 20.8 against 26.7; 9 in 3: 2048
-    // rows, 4.5 per CU, 68.3 against 67.4).  Key splits up to eight columns per
-    // CU (16 heads, 2048 rows: 79.7 us, paired 81.4, f32 109.9; 3000 rows: 152,
-    // 139, 201), paired blocks up to sixteen (32 heads, 2048 rows: 106 us,
-    // consecutive 112, f32 150; 3000 rows: 214, 200, 312).
-    if (head_dim == 64 && cols >= 3L * cus)
+    if (head_dim == 64 && hd64_splits(cols, cus, start, n))
         return cols <= 8L * cus    ? PrefillKernel::kSplitKeys
                : cols <= 16L * cus ? PrefillKernel::kSplitPaired
                                    : PrefillKernel::kSplitConsecutive;

@@ -192,8 +192,9 @@ def split_form(dim, heads, kv_heads, start, n, cus=256):
     """Which form of the split-bf16 kernel a prefill takes, or None.  With cols
     (head, 16-row block) columns: hd 128 from 128 keys on, but for the batches
     of paired_one_head, with key splits up to four columns per CU and paired
-    blocks up to eight; hd 64 from three columns per CU, with key splits up to
-    eight and paired blocks up to sixteen."""
+    blocks up to eight; hd 64 from three columns per CU, and the more of them
+    (weighted by the share of its keys that the average row sees) the longer the
+    history, with key splits up to eight and paired blocks up to sixteen."""
     hd = dim // heads
     cols = -(-n // 16) * heads
     if hd == 128:
@@ -201,7 +202,9 @@ def split_form(dim, heads, kv_heads, start, n, cus=256):
             return None
         keys, paired = 4, 8
     elif hd == 64:
-        if cols < 3 * cus:
+        seen = cols * (start + n / 2) / (start + n) / cus
+        if cols < 3 * cus or seen < (2.2 - 768 / (start + n) if cols <= 4 * cus else
+                                     min(2.5, 3 - 1280 / (start + n))):
             return None
         keys, paired = 8, 16
     else:

@@ -226,6 +226,19 @@ def test_prefill_plan_agrees_with_the_restated_rules(prefill_plan):
         assert (k == "paired_four_heads") == paired_register(dim, heads, kvh, start, n, cus), case
 
 
+def test_prefill_plan_leaves_long_batches_of_few_hd64_heads_to_f32(prefill_plan):
+    # (heads, kv_mul, start, n): batches that the split-bf16 kernel took 3 to 31%
+    # longer for, and some around them that it is faster at
+    slower = [(4, 4, 0, 3072), (4, 1, 0, 3277), (6, 3, 0, 2048), (4, 4, 600, 3072),
+              (8, 4, 0, 1536), (8, 4, 0, 1792), (8, 4, 0, 2099), (9, 3, 0, 1365),
+              (10, 2, 0, 1229), (9, 3, 0, 1866), (6, 3, 600, 2799), (6, 3, 0, 3072)]
+    faster = [(32, 4, 0, 384), (16, 4, 0, 1024), (15, 3, 0, 819), (8, 4, 600, 1536),
+              (14, 7, 0, 1200), (6, 3, 0, 2662), (8, 4, 0, 2560), (9, 3, 2000, 2048),
+              (6, 3, 600, 3072), (32, 4, 8000, 384)]
+    got = prefill_plan([(64, h, m, 256, start, n) for h, m, start, n in slower + faster])
+    assert got == ["key_split"] * len(slower) + ["split_keys"] * len(faster)
+
+
 def test_dispatch_sweep_reaches_every_prefill_kernel(prefill_plan):
     # the GPU sweep's targeted batches take the kernels they name on a 256-CU
     # device, and together reach every prefill kernel

@@ -313,9 +313,9 @@ def test_decode_large_scores_closed_form(name, p):
 # at 480; hd 128 MHA its consecutive form at 2048 rows and the f32 kernel of one
 # head, paired blocks and four key splits at 256.  The others run on f32: four
 # heads per workgroup at hd 256 and (paired) 32, one head and four query blocks
-# for hd 96 MHA; hd 48 and hd 16 give under two workgroups per CU at these
-# lengths and take the one-head kernel with the key tiles split over four
-# waves; 2048 rows of hd 64 in nine heads the split-bf16 one with key splits
+# for hd 96 MHA; the hd 64 (three heads), hd 48 and hd 16 shapes give under two
+# workgroups per CU at these lengths and take the one-head kernel with the key
+# tiles split over four waves
 PREFILL_CASES = [("llama3-8b", 0, 4096), ("llama3-8b", 24, 1000), ("llama3-8b", 100, 480),
                  ("hd128-mha", 40, 256), ("smollm2", 0, 2048),
                  ("stories15m", 0, 512), ("hd128-mha", 0, 2048), ("hd256-gqa4", 24, 1000),
