@@ -138,7 +138,12 @@ constexpr int prefill_waves_per_simd() {
 // waves are numbered key split first, then head, then block: the waves of one
 // SIMD hold the same head and key split of the heavy and the light block,
 // and every SIMD gets the same share.
-template <int HD, int HW, int QS, int NQT, int KSP, bool PAIR>
+//
+// APPEND: the workgroup first appends the batch's rows of its KV head
+// (prefill_appends()); kernels of their own, since the code ahead of the loop
+// cost the batches that do not append up to 3% (4 heads of 64, 3781 rows: 98.8
+// -> 101.9 us).
+template <int HD, int HW, int QS, int NQT, int KSP, bool PAIR, bool APPEND>
 __global__ __launch_bounds__(64 * HW * QS * KSP, (prefill_waves_per_simd<HD, HW>())) void
 prefill_mfma_kernel(PrefillParams p) {
     constexpr int kKT = 32;
@@ -213,7 +218,7 @@ prefill_mfma_kernel(PrefillParams p) {
 
     // The batch's rows of this KV head into the cache (prefill_appends(): the
     // only workgroup that writes or reads them), as kv_append_kernel does.
-    if (p.k_new != nullptr) {
+    if constexpr (APPEND) {
         for (int i = tid; i < p.n * (HD / 2); i += NT) {
             const int r = i / (HD / 2), j = i % (HD / 2);
             const long at = (long)r * p.kv_dim + g * HD + 2 * j;
@@ -626,7 +631,7 @@ prefill_mfma_kernel(PrefillParams p) {
     }
 }
 
-template <int HD, int HW, int QS, int KSP, bool PAIR = false>
+template <int HD, int HW, int QS, int KSP, bool PAIR = false, bool APPEND = false>
 hipError_t launch_t(const Shape& s, const PrefillParams& pp, hipStream_t st) {
     // 16 query rows per wave: measured on MI355X (hd 128, 4096 rows) 57% of
     // the fp32 MFMA peak against 47% with 32 rows per wave, because the lower
@@ -635,7 +640,7 @@ hipError_t launch_t(const Shape& s, const PrefillParams& pp, hipStream_t st) {
     constexpr int QB = 16 * NQT * QS;
     const int n_qb = PAIR ? ((pp.n + 15) / 16 + 1) / 2 : (pp.n + QB - 1) / QB;
     const dim3 grid(n_qb * (s.num_heads / HW));
-    hipLaunchKernelGGL((prefill_mfma_kernel<HD, HW, QS, NQT, KSP, PAIR>),
+    hipLaunchKernelGGL((prefill_mfma_kernel<HD, HW, QS, NQT, KSP, PAIR, APPEND>),
                        grid, dim3(64 * HW * QS * KSP), 0, st, pp);
     return hipGetLastError();
 }
@@ -643,11 +648,20 @@ hipError_t launch_t(const Shape& s, const PrefillParams& pp, hipStream_t st) {
 template <int HD>
 hipError_t launch_hd(const Shape& s, const PrefillParams& pp, PrefillKernel kernel,
                      hipStream_t st) {
+    const bool append = pp.k_new != nullptr;  // prefill_appends(): one of the first four
     switch (kernel) {
-        case PrefillKernel::kFourHeads: return launch_t<HD, 4, 1, 1>(s, pp, st);
-        case PrefillKernel::kThreeHeads: return launch_t<HD, 3, 1, 1>(s, pp, st);
-        case PrefillKernel::kTwoHeads: return launch_t<HD, 2, 2, 1>(s, pp, st);
-        case PrefillKernel::kOneHead: return launch_t<HD, 1, 4, 1>(s, pp, st);
+        case PrefillKernel::kFourHeads:
+            return append ? launch_t<HD, 4, 1, 1, false, true>(s, pp, st)
+                          : launch_t<HD, 4, 1, 1>(s, pp, st);
+        case PrefillKernel::kThreeHeads:
+            return append ? launch_t<HD, 3, 1, 1, false, true>(s, pp, st)
+                          : launch_t<HD, 3, 1, 1>(s, pp, st);
+        case PrefillKernel::kTwoHeads:
+            return append ? launch_t<HD, 2, 2, 1, false, true>(s, pp, st)
+                          : launch_t<HD, 2, 2, 1>(s, pp, st);
+        case PrefillKernel::kOneHead:
+            return append ? launch_t<HD, 1, 4, 1, false, true>(s, pp, st)
+                          : launch_t<HD, 1, 4, 1>(s, pp, st);
         case PrefillKernel::kKeySplit:
             if constexpr (HD <= 64) return launch_t<HD, 1, 1, 4>(s, pp, st);
             break;
