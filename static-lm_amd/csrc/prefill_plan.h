@@ -156,10 +156,15 @@ inline PrefillKernel prefill_plan(int head_dim, int num_heads, int kv_mul, int c
 // group, all heads of the KV head), so that each row has one writer and every
 // reader of a new row is in its workgroup: batches of at most 16 rows (four or
 // three heads per KV head), 32 (two) or 64 (one).  It saves the append launch,
-// which takes as long as such a batch's attention (16 rows of 6
-// heads of 48, per call: 6.8 us appended apart, 4.1 inside).
+// which takes as long as such a batch's attention (16 rows of 6 heads of 48, per
+// call: 7.1 us appended apart, 4.6 inside), but few workgroups then wait for all
+// the rows: up to 2560 values of K and V each per KV head.  Apart against
+// inside, 6 heads without GQA: hd 48, 48 / 56 rows 7.2 / 7.3 against 7.1 / 7.5 us;
+// hd 64, 40 / 64 rows 7.7 / 8.1 against 7.2 / 8.5; hd 96, 24 / 33 rows 7.3 / 9.2
+// against 7.0 / 9.7; hd 128, 17 / 24 / 64 rows 8.0 / 8.2 / 11.6 against 7.5 / 8.1 /
+// 14.7; hd 256, 8 / 16 / 64 rows 11.2 / 11.7 / 19.1 against 10.6 / 12.2 / 26.5.
 inline bool prefill_appends(int head_dim, int num_heads, int kv_mul, int cus, int start, int n) {
-    if (n < 2) return false;
+    if (n < 2 || (long)n * head_dim > 2560) return false;
     const PrefillTiling t = prefill_tiling(kv_mul);
     const PrefillKernel k = prefill_plan(head_dim, num_heads, kv_mul, cus, start, n);
     return t.hw == kv_mul && n <= 16 * t.qs &&

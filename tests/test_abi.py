@@ -239,6 +239,25 @@ def test_prefill_plan_leaves_long_batches_of_few_hd64_heads_to_f32(prefill_plan)
     assert got == ["key_split"] * len(slower) + ["split_keys"] * len(faster)
 
 
+def test_prefill_appends_only_what_few_workgroups_take_quickly(tmp_path):
+    # (hd, heads, kv_mul, start, n): batches whose attention kernel appends the
+    # rows itself, and larger ones, where the append launch is faster (1.02 to
+    # 1.39 times the time inside)
+    inside = [(48, 6, 1, 0, 16), (48, 6, 1, 0, 53), (64, 6, 1, 40, 40), (96, 6, 1, 0, 26),
+              (128, 16, 2, 0, 20), (256, 6, 1, 0, 10), (128, 32, 4, 0, 16), (16, 6, 1, 40, 64)]
+    apart = [(48, 6, 1, 0, 64), (64, 6, 1, 0, 64), (96, 6, 1, 0, 33), (128, 6, 1, 0, 64),
+             (256, 6, 1, 0, 64), (256, 9, 3, 0, 16), (256, 4, 2, 40, 32), (128, 16, 2, 0, 32),
+             (48, 6, 1, 0, 65), (128, 32, 4, 0, 17), (48, 6, 1, 0, 1)]
+    src = tmp_path / "appends.cpp"
+    src.write_text(PLAN_PROBE.replace("(int)slm::prefill_plan(", "(int)slm::prefill_appends("))
+    exe = tmp_path / "appends"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror",
+                    f"-I{P.PKG_DIR / 'csrc'}", str(src), "-o", str(exe)], check=True)
+    inp = "".join(f"{hd} {h} {m} 256 {start} {n}\n" for hd, h, m, start, n in inside + apart)
+    out = subprocess.run([str(exe)], input=inp, capture_output=True, text=True, check=True).stdout
+    assert out.split() == ["1"] * len(inside) + ["0"] * len(apart)
+
+
 def test_dispatch_sweep_reaches_every_prefill_kernel(prefill_plan):
     # the GPU sweep's targeted batches take the kernels they name on a 256-CU
     # device, and together reach every prefill kernel

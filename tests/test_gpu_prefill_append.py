@@ -15,6 +15,9 @@ CASES = [
     (128, 8, 2, 0, 2), (128, 8, 2, 60, 15), (128, 8, 2, 3, 16), (128, 8, 2, 3, 17),
     (64, 9, 3, 0, 16), (64, 9, 3, 31, 17), (16, 6, 2, 9, 16), (256, 4, 1, 16, 16),
     (32, 4, 2, 0, 31), (96, 4, 2, 1, 32), (96, 4, 2, 1, 33),
+    (96, 4, 2, 1, 26), (96, 4, 2, 1, 27), (128, 4, 2, 0, 20), (128, 4, 2, 0, 21),
+    (256, 2, 2, 5, 10), (256, 2, 2, 5, 11), (64, 2, 2, 3, 40), (64, 2, 2, 3, 41),
+    (48, 6, 6, 0, 53), (48, 6, 6, 0, 54), (32, 4, 4, 9, 64),
     (48, 6, 6, 0, 16), (48, 6, 6, 7, 63), (16, 4, 4, 0, 64), (48, 6, 6, 0, 65), (256, 2, 2, 5, 64),
 ]
 
