@@ -776,10 +776,17 @@ __device__ __forceinline__ float sum_f32(int d) {
 // 4330 us; dim 576, hidden 1536, 130 / 512 tokens 56 -> 53, 73 -> 70; dim 288,
 // hidden 768, 300 tokens 52 -> 47.  (The exp's VALU work in the epilogue takes
 // back about half of what the memory traffic cost.)
-template <int WRW, int WTW, int NTS, bool ACT>
+//
+// PIPE (one MFMA per wave and block): nothing else covers an MFMA's latency where
+// a CU has at most one workgroup, so the next block's is issued early: 4096 x
+// 14336, 100 / 256 tokens 117 / 120 -> 111 / 114 us, 14336 x 4096, 32 tokens 37.0 ->
+// 35.3; with more workgroups they cover it better themselves (4096 x 14336, 300
+// tokens 136 against 143 so).
+template <int WRW, int WTW, int NTS, bool PIPE, bool ACT>
 __global__ __launch_bounds__(64 * WRW * WTW) void gemm_q4_mfma_kernel(GemmParams p) {
 #pragma clang fp contract(off)
     using Sh = GemmShape<WRW, WTW, NTS>;
+    static_assert(!PIPE || NTS == 1, "one product per block");
     constexpr int RT = Sh::RT, TT = Sh::TT;
     __shared__ __align__(16) GemmStage<RT, TT> st[2];
     const int tid = threadIdx.x;
@@ -901,18 +908,28 @@ __global__ __launch_bounds__(64 * WRW * WTW) void gemm_q4_mfma_kernel(GemmParams
         if (sg + 1 < n_stages) SLM_GEMM_LOAD_STAGE((sg + 1) * kScaleChunk);
         const GemmStage<RT, TT>& S = st[sg & 1];
         const int b0 = sg * kScaleChunk;
+        auto product = [&](int kb, int s) __attribute__((always_inline)) {
+            const v4i af = *reinterpret_cast<const v4i*>(
+                &S.a[(qr + l32) * kAStride + kb * 8 + 4 * hh]);
+            const v4i bf = *reinterpret_cast<const v4i*>(
+                &S.b[(qt + 32 * s + l32) * kBStride + kb * 8 + 4 * hh]);
+            return __builtin_amdgcn_mfma_i32_32x32x32_i8(af, bf, base, 0, 0, 0);
+        };
+        // PIPE: the next block's MFMA is issued ahead of this one's epilogue
+        // (past the row's last block: of stale bytes, and unused).
+        v16i d[NTS], next;
+        if constexpr (PIPE) next = product(0, 0);
 #pragma unroll
         for (int kb = 0; kb < kScaleChunk; ++kb) {
             if (b0 + kb >= nb) break;  // uniform
-            const v4i af = *reinterpret_cast<const v4i*>(
-                &S.a[(qr + l32) * kAStride + kb * 8 + 4 * hh]);
-            v16i d[NTS];
             float da[NTS];
+            if constexpr (PIPE) {
+                d[0] = next;
+                if (kb + 1 < kScaleChunk) next = product(kb + 1, 0);
+            }
 #pragma unroll
             for (int s = 0; s < NTS; ++s) {
-                const v4i bf = *reinterpret_cast<const v4i*>(
-                    &S.b[(qt + 32 * s + l32) * kBStride + kb * 8 + 4 * hh]);
-                d[s] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, bf, base, 0, 0, 0);
+                if constexpr (!PIPE) d[s] = product(kb, s);
                 da[s] = S.da[kb][qt + 32 * s + l32];
             }
             // the scale products stay on the VALU: on the matrix cores (an
@@ -979,33 +996,48 @@ __global__ __launch_bounds__(64 * WRW * WTW) void gemm_q4_mfma_kernel(GemmParams
                       15) == 0;
     const int rb = wr0 + qr + 4 * hh;  // this lane's rows: rb + 8a + (0..3)
     if (vec) {
+        // Lanes l and l ^ 1 swap row groups first, so that one access covers 64
+        // bytes of 16 tokens instead of 32 of 32: access a takes token a & 1 of
+        // the pair and rows 8 ((a & 2) + (l & 1)) .. of the wave (16384 x 64, 1024
+        // tokens 26.2 -> 22.8 us; 32000 x 288, 512 tokens 42.2 -> 38.0).
+        const int odd = lane & 1;
+        auto tok = [&](int s, int a) { return wt0 + qt + 32 * s + (l32 & ~1) + (a & 1); };
+        auto row = [&](int a) { return rb + 8 * ((a & 2) + odd); };
         float4 rv[NTS][4];
         if (M.res) {
 #pragma unroll
             for (int s = 0; s < NTS; ++s)
 #pragma unroll
                 for (int a = 0; a < 4; ++a) {
-                    const int t = min(wt0 + qt + 32 * s + l32, p.batch - 1);
-                    const int r0 = min(rb + 8 * a, M.rows - 4);
+                    const int t = min(tok(s, a), p.batch - 1);
+                    const int r0 = min(row(a), M.rows - 4);
                     rv[s][a] = ld4(M.res + (long)t * M.out_stride + r0);
                 }
         }
 #pragma unroll
         for (int s = 0; s < NTS; ++s)
 #pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                const int t = wt0 + qt + 32 * s + l32;
-                const int r0 = rb + 8 * a;
-                if (t >= p.batch || r0 >= M.rows) continue;
-                float4 y = make_float4(acc[s][4 * a], acc[s][4 * a + 1], acc[s][4 * a + 2],
-                                       acc[s][4 * a + 3]);
-                if (M.res) {
-                    y.x = rv[s][a].x + y.x;
-                    y.y = rv[s][a].y + y.y;
-                    y.z = rv[s][a].z + y.z;
-                    y.w = rv[s][a].w + y.w;
+            for (int h = 0; h < 4; h += 2) {
+                float4 y[2];  // of the pair's first and second token
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float lo = acc[s][4 * h + r], hi = acc[s][4 * h + 4 + r];
+                    const float got = dpp<0xB1>(odd ? lo : hi);  // quad_perm [1,0,3,2]
+                    (&y[0].x)[r] = odd ? got : lo;
+                    (&y[1].x)[r] = odd ? hi : got;
                 }
-                *reinterpret_cast<float4*>(M.out + (long)t * M.out_stride + r0) = y;
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const int t = tok(s, h + i), r0 = row(h + i);
+                    if (t >= p.batch || r0 >= M.rows) continue;
+                    if (M.res) {
+                        y[i].x = rv[s][h + i].x + y[i].x;
+                        y[i].y = rv[s][h + i].y + y[i].y;
+                        y[i].z = rv[s][h + i].z + y[i].z;
+                        y[i].w = rv[s][h + i].w + y[i].w;
+                    }
+                    *reinterpret_cast<float4*>(M.out + (long)t * M.out_stride + r0) = y[i];
+                }
             }
         return;
     }
@@ -1349,19 +1381,19 @@ unsigned gemm_params(const Q4Job* jobs, int njobs, const uint32_t* aq, const flo
     return grid > 0x7FFFFFFF ? 0 : (unsigned)grid;
 }
 
-template <int WRW, int WTW, int NTS>
+template <int WRW, int WTW, int NTS, bool PIPE>
 hipError_t launch_gemm_t(const Q4Job* jobs, int njobs, const uint32_t* aq, const float* ad,
                          int nb, int batch, hipStream_t st) {
     using Sh = GemmShape<WRW, WTW, NTS>;
     GemmParams p;
     const unsigned grid = gemm_params(jobs, njobs, aq, ad, nb, batch, Sh::RT, Sh::TT, &p);
     if (!grid) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((gemm_q4_mfma_kernel<WRW, WTW, NTS, false>), dim3(grid), dim3(Sh::NT), 0,
-                       st, p);
+    hipLaunchKernelGGL((gemm_q4_mfma_kernel<WRW, WTW, NTS, PIPE, false>), dim3(grid),
+                       dim3(Sh::NT), 0, st, p);
     return hipGetLastError();
 }
 
-template <int WRW, int WTW, int NTS>
+template <int WRW, int WTW, int NTS, bool PIPE>
 hipError_t launch_gemm_swiglu_t(const Q4Job& gate, const Q4Job& up, const uint32_t* aq,
                                 const float* ad, int nb, int batch, const Q8Out& act,
                                 hipStream_t st) {
@@ -1372,8 +1404,8 @@ hipError_t launch_gemm_swiglu_t(const Q4Job& gate, const Q4Job& up, const uint32
     if (!grid) return hipErrorInvalidValue;
     p.m[1] = QMat{up.qs, up.d, up.out, up.res, up.rows, up.out_stride, q4_scale_stride(nb)};
     p.act = act;
-    hipLaunchKernelGGL((gemm_q4_mfma_kernel<WRW, WTW, NTS, true>), dim3(grid), dim3(Sh::NT), 0,
-                       st, p);
+    hipLaunchKernelGGL((gemm_q4_mfma_kernel<WRW, WTW, NTS, PIPE, true>), dim3(grid),
+                       dim3(Sh::NT), 0, st, p);
     return hipGetLastError();
 }
 
@@ -1477,7 +1509,7 @@ long device_cus() {
 // would leave CUs idle (Wo at 512 tokens: 128 workgroups of 128 x 128 on 256
 // CUs).  Tile shape does not change results (each output is one thread's
 // ordered sum over blocks).
-enum class GemmForm { kSmall, k64, k128 };
+enum class GemmForm { kSmall, k64Few, k64, k128 };
 
 GemmForm gemm_form(const Q4Job* jobs, int njobs, int batch) {
     long w128 = 0, w64 = 0, w16 = 0;
@@ -1491,7 +1523,8 @@ GemmForm gemm_form(const Q4Job* jobs, int njobs, int batch) {
     if (w16 <= 4 * cus) return GemmForm::kSmall;
     const double t128 = (double)((w128 + cus - 1) / cus) * 4.0;
     const double t64 = (double)((w64 + cus - 1) / cus) * 1.1;
-    return t128 < t64 ? GemmForm::k128 : GemmForm::k64;
+    if (t128 < t64) return GemmForm::k128;
+    return w64 <= cus ? GemmForm::k64Few : GemmForm::k64;
 }
 
 }  // namespace
@@ -1501,10 +1534,13 @@ hipError_t launch_q4_gemm(const Q4Job* jobs, int njobs, const uint32_t* aq, cons
     if (njobs < 1 || njobs > 3 || batch < 1) return hipErrorInvalidValue;
     switch (gemm_form(jobs, njobs, batch)) {
         case GemmForm::kSmall: return launch_gemm_small(jobs, njobs, aq, ad, nb, batch, st);
-        case GemmForm::k128: return launch_gemm_t<4, 2, 2>(jobs, njobs, aq, ad, nb, batch, st);
+        case GemmForm::k64Few:
+            return launch_gemm_t<2, 2, 1, true>(jobs, njobs, aq, ad, nb, batch, st);
+        case GemmForm::k128:
+            return launch_gemm_t<4, 2, 2, false>(jobs, njobs, aq, ad, nb, batch, st);
         case GemmForm::k64: break;
     }
-    return launch_gemm_t<2, 2, 1>(jobs, njobs, aq, ad, nb, batch, st);
+    return launch_gemm_t<2, 2, 1, false>(jobs, njobs, aq, ad, nb, batch, st);
 }
 
 bool q4_gemm_takes_swiglu(const Q4Job& gate, const Q4Job& up, int batch) {
@@ -1518,9 +1554,13 @@ hipError_t launch_q4_gemm_swiglu(const Q4Job& gate, const Q4Job& up, const uint3
                                  hipStream_t st) {
     if (!q4_gemm_takes_swiglu(gate, up, batch)) return hipErrorInvalidValue;
     const Q4Job jobs[2] = {gate, up};
-    return gemm_form(jobs, 2, batch) == GemmForm::k128
-               ? launch_gemm_swiglu_t<4, 2, 2>(gate, up, aq, ad, nb, batch, act, st)
-               : launch_gemm_swiglu_t<2, 2, 1>(gate, up, aq, ad, nb, batch, act, st);
+    switch (gemm_form(jobs, 2, batch)) {
+        case GemmForm::k128:
+            return launch_gemm_swiglu_t<4, 2, 2, false>(gate, up, aq, ad, nb, batch, act, st);
+        case GemmForm::k64Few:
+            return launch_gemm_swiglu_t<2, 2, 1, true>(gate, up, aq, ad, nb, batch, act, st);
+        default: return launch_gemm_swiglu_t<2, 2, 1, false>(gate, up, aq, ad, nb, batch, act, st);
+    }
 }
 
 }  // namespace slm

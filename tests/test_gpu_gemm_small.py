@@ -1,6 +1,6 @@
 """The Q4_0 GEMM whose blocks are split over the waves, at the edges of its
-16 x 16 tiles, its 4-block and 32-block steps and its dispatch, bit for bit
-against the scalar oracle."""
+16 x 16 tiles, its 4-block and 32-block steps and its dispatch, and the tiled
+forms, bit for bit against the scalar oracle."""
 import numpy as np
 import pytest
 
@@ -53,6 +53,18 @@ def test_bit_exact_with_scalar_reference(ctx, rows, cols, batch, residual):
     if residual:
         want = res + want
     assert_bitwise(got, want, f"gemm {rows}x{cols} batch {batch}")
+
+
+# the tiled forms: 64 x 64 tiles at most one per CU and more, 128 x 128 tiles;
+# whole and ragged tiles, rows in fours and not, one and two stages of blocks
+TILED = [(1024, 64, 320), (1028, 96, 301), (1028, 288, 290), (1027, 64, 301), (4096, 64, 320),
+         (4100, 64, 257), (4099, 288, 263), (8192, 64, 512), (8188, 64, 509), (8189, 288, 509)]
+
+
+@pytest.mark.parametrize("rows,cols,batch", TILED)
+@pytest.mark.parametrize("residual", [False, True])
+def test_tiles_bit_exact_with_scalar_reference(ctx, rows, cols, batch, residual):
+    test_bit_exact_with_scalar_reference(ctx, rows, cols, batch, residual)
 
 
 def test_infinite_scales(ctx):
