@@ -1499,7 +1499,10 @@ long device_cus() {
 // workgroups) 35 / 35 / 36 / 37 against 11 / 17 / 28 / 48 us; 4096 x 14336, 16 / 64
 // tokens 111 / 113 against 29 / 80; 14336 x 4096, 16 / 32 tokens (896 / 1792) 35.7 /
 // 36.2 against 27 / 43; 576 x 1536, 130 / 512 tokens (324 / 1152) 17.2 / 17.8 against
-// 10.1 / 18.7.
+// 10.1 / 18.7.  Short rows leave little to split: with two stages of blocks (9 to
+// 16) it is ahead up to 2.5 per CU (1024 x 384, 160 / 224 tokens 8.6 / 8.5 against
+// 8.7 / 9.8; x 512 9.4 / 9.4 against 9.0 / 9.8), with one it never is (1024 x 256,
+// 64 / 128 / 256 tokens 7.1 / 7.4 / 7.5 against 7.4 / 7.5 / 9.7).
 //
 // Otherwise 128 x 128 workgroups (one per CU; less VALU per output element and
 // block) or 64 x 64 (two per CU).  On 32x32x32 MFMAs (against 16x16x32 ones, which
@@ -1511,7 +1514,7 @@ long device_cus() {
 // ordered sum over blocks).
 enum class GemmForm { kSmall, k64Few, k64, k128 };
 
-GemmForm gemm_form(const Q4Job* jobs, int njobs, int batch) {
+GemmForm gemm_form(const Q4Job* jobs, int njobs, int nb, int batch) {
     long w128 = 0, w64 = 0, w16 = 0;
     for (int i = 0; i < njobs; ++i) {
         w128 += (long)((jobs[i].rows + 127) / 128) * ((batch + 127) / 128);
@@ -1520,7 +1523,8 @@ GemmForm gemm_form(const Q4Job* jobs, int njobs, int batch) {
                ((batch + kSmallToks - 1) / kSmallToks);
     }
     const long cus = device_cus();
-    if (w16 <= 4 * cus) return GemmForm::kSmall;
+    const long stages = (nb + kScaleChunk - 1) / kScaleChunk;
+    if (stages > 1 && 2 * w16 <= (stages == 2 ? 5 : 8) * cus) return GemmForm::kSmall;
     const double t128 = (double)((w128 + cus - 1) / cus) * 4.0;
     const double t64 = (double)((w64 + cus - 1) / cus) * 1.1;
     if (t128 < t64) return GemmForm::k128;
@@ -1532,7 +1536,7 @@ GemmForm gemm_form(const Q4Job* jobs, int njobs, int batch) {
 hipError_t launch_q4_gemm(const Q4Job* jobs, int njobs, const uint32_t* aq, const float* ad,
                           int nb, int batch, hipStream_t st) {
     if (njobs < 1 || njobs > 3 || batch < 1) return hipErrorInvalidValue;
-    switch (gemm_form(jobs, njobs, batch)) {
+    switch (gemm_form(jobs, njobs, nb, batch)) {
         case GemmForm::kSmall: return launch_gemm_small(jobs, njobs, aq, ad, nb, batch, st);
         case GemmForm::k64Few:
             return launch_gemm_t<2, 2, 1, true>(jobs, njobs, aq, ad, nb, batch, st);
@@ -1543,18 +1547,18 @@ hipError_t launch_q4_gemm(const Q4Job* jobs, int njobs, const uint32_t* aq, cons
     return launch_gemm_t<2, 2, 1, false>(jobs, njobs, aq, ad, nb, batch, st);
 }
 
-bool q4_gemm_takes_swiglu(const Q4Job& gate, const Q4Job& up, int batch) {
+bool q4_gemm_takes_swiglu(const Q4Job& gate, const Q4Job& up, int nb, int batch) {
     const Q4Job jobs[2] = {gate, up};
     return gate.rows == up.rows && gate.rows % 32 == 0 && batch >= 1 &&
-           gemm_form(jobs, 2, batch) != GemmForm::kSmall;
+           gemm_form(jobs, 2, nb, batch) != GemmForm::kSmall;
 }
 
 hipError_t launch_q4_gemm_swiglu(const Q4Job& gate, const Q4Job& up, const uint32_t* aq,
                                  const float* ad, int nb, int batch, const Q8Out& act,
                                  hipStream_t st) {
-    if (!q4_gemm_takes_swiglu(gate, up, batch)) return hipErrorInvalidValue;
+    if (!q4_gemm_takes_swiglu(gate, up, nb, batch)) return hipErrorInvalidValue;
     const Q4Job jobs[2] = {gate, up};
-    switch (gemm_form(jobs, 2, batch)) {
+    switch (gemm_form(jobs, 2, nb, batch)) {
         case GemmForm::k128:
             return launch_gemm_swiglu_t<4, 2, 2, false>(gate, up, aq, ad, nb, batch, act, st);
         case GemmForm::k64Few:

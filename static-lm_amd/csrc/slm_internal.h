@@ -157,7 +157,7 @@ hipError_t launch_q4_gemm(const Q4Job* jobs, int njobs, const uint32_t* aq, cons
 // gate and up with SwiGLU fused: Q8_0 blocks of silu(gate . x) * (up . x), no
 // block sums; for the batches that q4_gemm_takes_swiglu names (the others have
 // so few tiles that the separate launches' split over the blocks is faster)
-bool q4_gemm_takes_swiglu(const Q4Job& gate, const Q4Job& up, int batch);
+bool q4_gemm_takes_swiglu(const Q4Job& gate, const Q4Job& up, int nb, int batch);
 hipError_t launch_q4_gemm_swiglu(const Q4Job& gate, const Q4Job& up, const uint32_t* aq,
                                  const float* ad, int nb, int batch, const Q8Out& act,
                                  hipStream_t st);

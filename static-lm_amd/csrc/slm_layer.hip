@@ -209,7 +209,7 @@ int slm_layer_forward_dev(slm_attn_ctx* c, int32_t layer, int32_t start, int32_t
     // (its input is still being read), or in a launch of its own
     slm::Q8Out act = q8_out(c, nbh);
     const slm::Q4Job gate = q4_job(w->w_gate, hb), up = q4_job(w->w_up, hb2);
-    if (slm::q4_gemm_takes_swiglu(gate, up, n)) {
+    if (slm::q4_gemm_takes_swiglu(gate, up, nb, n)) {
         act.q = reinterpret_cast<uint32_t*>(hb);  // n * hidden bytes
         act.d = hb2;  // n * d_stride floats, at most n * hidden
         Timed t(c, SLM_K_GEMM);

@@ -34,12 +34,14 @@ def product(ctx, w, rows, cols, x, res=None):
         return out.cpu().numpy()
 
 
-# rows, cols, batch: ragged row and token tiles; 1, 4, 5, 31 to 33, 64, 65 and
-# 512 blocks; the last batch of 1024 rows that is split (64 x 16 workgroups on
-# 256 CUs) and the first that is tiled
-CASES = [(16, 32, 5), (20, 128, 16), (33, 160, 15), (7, 992, 17), (48, 1024, 33), (31, 1056, 6),
-         (64, 2048, 7), (65, 2080, 48), (96, 16384, 9), (1024, 64, 256), (1024, 64, 257),
-         (4096, 4096, 12)]
+# rows, cols, batch: ragged row and token tiles; 9, 12, 13, 31 to 33, 64, 65 and
+# 512 blocks; the last batches of 1024 rows that are split (64 x 10 workgroups of
+# up to 16 blocks, 64 x 16 of more, on 256 CUs) and the first that are tiled;
+# rows of 1 to 8 blocks, which are always tiled
+CASES = [(20, 288, 16), (33, 384, 15), (24, 416, 5), (7, 992, 17), (48, 1024, 33), (31, 1056, 6),
+         (64, 2048, 7), (65, 2080, 48), (96, 16384, 9), (1024, 512, 160), (1024, 512, 161),
+         (1024, 544, 256), (1024, 544, 257), (4096, 4096, 12),
+         (16, 32, 5), (20, 128, 16), (33, 160, 15), (48, 256, 33), (1024, 64, 256), (1024, 64, 257)]
 
 
 @pytest.mark.parametrize("rows,cols,batch", CASES)

@@ -11,11 +11,14 @@ P = load_product()
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
-# dim, hidden, n, weight scale: the last batch of separate launches and the
-# first fused one (128, 129 tokens of hidden 1024), 64 x 64 tiles with hidden
-# and tokens cut by a tile, one block of nine more than a stage, 128 x 128 tiles
-# whole and cut, and gates large enough to saturate
+# dim, hidden, n, weight scale: the last batches of separate launches and the
+# first fused ones (80, 81 tokens of hidden 1024 at 9 blocks, 128, 129 at 17), the
+# smallest fused one, 64 x 64 tiles with hidden and tokens cut by a tile, one
+# block of nine more than a stage, 128 x 128 tiles whole and cut, and gates large
+# enough to saturate
 CASES = [
+    (288, 1024, 80, 0.3), (288, 1024, 81, 0.3), (544, 1024, 128, 0.3), (544, 1024, 129, 0.3),
+    (64, 32, 2, 0.3), (256, 704, 33, 0.3),
     (128, 1024, 128, 0.3), (128, 1024, 129, 0.3), (64, 1056, 193, 0.3), (288, 1568, 160, 0.3),
     (128, 4096, 512, 0.3), (128, 4064, 385, 0.3), (320, 4064, 500, 30.0), (64, 1056, 255, 30.0),
 ]
