@@ -211,7 +211,8 @@ int slm_rope_tables_read(slm_attn_ctx* ctx, float* cos_out, float* sin_out);
  * recorded around the launch, which adds its dispatch (~2 us).
  * Reading resets the counters. */
 enum {
-    SLM_K_APPEND = 0,  /* rope(k) + KV append of a prefill batch */
+    SLM_K_APPEND = 0,  /* rope(k) + KV append of a prefill batch (the smallest batches append
+                        * in their attention kernel: SLM_K_PREFILL) */
     SLM_K_DECODE = 1,  /* decode: in-kernel KV append + split-K attention */
     SLM_K_COMBINE = 2, /* merge of the decode split partials */
     SLM_K_PREFILL = 3, /* causal prefill attention */
@@ -219,7 +220,8 @@ enum {
     SLM_K_QUANT = 5,   /* Q8_0 activation quantization (slm_quant.h) */
     SLM_K_GEMM = 6,    /* Q4_0 x Q8_0 GEMV / GEMM (slm_quant.h) */
     SLM_K_NORM = 7,    /* RMSNorm / L2 norm (slm_layer.h) */
-    SLM_K_ELEM = 8,    /* SwiGLU, residual add, embedding rows, argmax (slm_layer.h) */
+    SLM_K_ELEM = 8,    /* SwiGLU (where its projection does not apply it: SLM_K_GEMM), residual
+                        * add, embedding rows, argmax (slm_layer.h) */
     SLM_K_COUNT = 9
 };
 typedef struct slm_kernel_stat {

@@ -23,7 +23,8 @@ HOST_DEMO = PKG_DIR / "slm_host_demo"
 BUILD_DIR = PKG_DIR / "_build"
 
 HIP_SOURCES = ["slm_attn.hip", "slm_layer.hip", "slm_model.hip", "rope_append.hip",
-               "attn_decode.hip", "prefill_mfma.hip", "prefill_split.hip", "quant_gemm.hip", "norm_act.hip"]
+               "attn_decode.hip", "prefill_mfma.hip", "prefill_split.hip", "quant_gemm.hip",
+               "norm_act.hip"]
 # measurement probes of the bench, a library of their own (not the product's)
 CALIB_DIR = PKG_DIR / "calib"
 CALIB_LIB = CALIB_DIR / "libslm_calib.so"
@@ -46,9 +47,9 @@ HIP_FLAGS = [
     f"-I{REPO / 'include'}",
     f"-I{CSRC}",
 ]
-# per-source extras: the Q4_0 GEMM's MFMA results go straight to VGPRs (its
-# epilogue reads every one; accumulator registers would cost a
-# v_accvgpr_read per element)
+# per-source extras: MFMA results of the Q4_0 GEMM and the split-bf16 prefill go
+# straight to VGPRs (their VALU work reads every one; accumulator registers
+# would cost a v_accvgpr_read per element)
 HIP_SOURCE_FLAGS = {"quant_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
                     "prefill_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 

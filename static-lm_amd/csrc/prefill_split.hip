@@ -7,17 +7,17 @@
 // Precision.  An f32 value is the sum of three bf16 values x1 + x2 + x3 (each
 // the rounded remainder of the ones before), so a product is nine bf16
 // products, exact in f32; x2*y3, x3*y2 and x3*y3 (below 2^-25 of the product)
-// are left out.  The five small products and the leading one are summed
-// apart, and the output accumulators take one addition per 32-key tile, so
-// fewer roundings at full magnitude go into a result than with
-// v_mfma_f32_16x16x4_f32, which adds four products at a time.
+// are left out.  The other six are added to the accumulator one after another,
+// small ones first: six roundings for 32 products, where
+// v_mfma_f32_16x16x4_f32 has eight (error against 64 bits at 4096 rows 7.1e-7,
+// in f32 8.6e-7).
 //
 // What bounds it: six bf16 products at 16 times the f32 MFMA rate.  A 16 x 32
-// x 128 product takes 48 MFMAs of 16 cycles against 64 of 32 for f32, and the
-// VALU work (softmax, splitting K, V and P) of one wave can run beside another
-// wave's MFMAs of a SIMD, which it cannot beside f32 MFMAs.
+// x 128 product takes 48 MFMAs of 16 cycles against 64 of 32 for f32; the VALU
+// work (softmax, splitting K, V and P) overlaps MFMAs of another wave of the
+// SIMD only in part, and at 4096 rows the matrix pipes are busy half the time.
 //
-// Tiling.  A workgroup holds HW query heads of one KV head, two blocks of 16
+// Tiling.  A workgroup holds HW query heads of one KV head, QS blocks of 16
 // query rows and KSP key splits, a wave for each; with PAIR the blocks are i
 // and n_blocks-1-i (every workgroup then has the same causal work), and the
 // waves are numbered key split first, then head, then block, so a SIMD holds
@@ -32,8 +32,9 @@
 //                    they never move between lanes and V is stored with its
 //                    keys in that order.
 // Each wave's share of the next tiles goes from memory into its own LDS bytes
-// by DMA, so no registers are held for it.  With 80 KiB of LDS (KSP 1) two
-// workgroups share a CU, and one's MFMAs run beside the other's splitting.
+// by DMA, so no registers are held for it.  At hd 128 the planes and raw bytes
+// take 128 KiB of LDS (160 with key splits), one workgroup and two waves per SIMD
+// for a CU; at hd 64 half of that, two workgroups.
 //
 // Values that cannot be split.  inf, and finite values that round to a bf16 inf,
 // make NaN when split, and the remainders of values below 2^-109 run out of
@@ -125,7 +126,6 @@ template <int HD, int HW, int QS, int KSP, bool PAIR>
 __global__ __launch_bounds__(64 * QS * HW * KSP, HD == 64 ? 4 : 2) void prefill_split_kernel(
     SplitParams p) {
     constexpr int NB = KSP == 1 ? 2 : 1;  // plane buffers
-    
     constexpr int NWS = QS * HW;       // waves of one key split
     constexpr int NW = NWS * KSP;
     constexpr int NT = 64 * NW;
@@ -142,8 +142,9 @@ __global__ __launch_bounds__(64 * QS * HW * KSP, HD == 64 ? 4 : 2) void prefill_
     // planes: dim d's chunk g (the keys lane group g supplies) in slot g ^
     // v_swz(d).  A 64-lane ds_read_b128 is served in four cycles of 16 lanes of
     // a half-wave that agree in the parity of lane bits 2-4 (bit 0 may also
-    // count); with these slots the 16 lanes of reads and stores cover the 64
-    // banks once, either way.
+    // count); with these slots the 16 lanes of the planes' reads and stores cover
+    // the 64 banks once, either way.  What conflicts are left (11% of the LDS
+    // cycles at 4096 rows) come with the raw K bytes, read 32 bytes apart.
     __shared__ __align__(16) struct {
         uint4 k[NB * KSP][3][PL];
         uint4 v[NB * KSP][3][PL];
@@ -458,8 +459,10 @@ __global__ __launch_bounds__(64 * QS * HW * KSP, HD == 64 ? 4 : 2) void prefill_
             __syncthreads();  // every wave is done with them
         }
     } else {
-        // Half of a SIMD's waves split the next tile before they attend this
-        // one, the others afterwards, so that splitting runs beside MFMAs.
+        // Half of the waves split the next tile before they attend this one,
+        // the others afterwards, so that splitting runs beside MFMAs: waves w and
+        // w + 4 share a SIMD, one of each with four heads per workgroup (with
+        // two or one both are alike).
         auto next = [&](int st, int buf) __attribute__((always_inline)) {
             if (st + 1 >= n_steps) return;
             stage(buf ^ 1);
